@@ -733,24 +733,38 @@ hipError_t launch_decode(const uint4* tiles, const uint2* sb, const uint16_t* x,
 
 // argmax over the blocks' best keys: one workgroup per row (deterministic: the max of
 // keys does not depend on order)
-__global__ __launch_bounds__(256) void greedy_reduce_kernel(const unsigned long long* __restrict__ part, int nb,
-                                                            int32_t* __restrict__ token, float* __restrict__ value) {
+// Latency-bound: one workgroup per row, each thread's kGreedyKeys keys all requested
+// before the first comparison (the lm_head's 16384 keys in one round trip; 256 threads
+// taking 64 keys one after another waited for most of them: 17 us, 3 us so).
+constexpr int kGreedyThreads = 1024;
+constexpr int kGreedyKeys = 16;
+__global__ __launch_bounds__(kGreedyThreads) void greedy_reduce_kernel(const unsigned long long* __restrict__ part,
+                                                                       int nb, int32_t* __restrict__ token,
+                                                                       float* __restrict__ value) {
     const int m = (int)blockIdx.x;
+    const unsigned long long* const keys = part + (long)m * nb;
     unsigned long long best = 0;
-    for (int i = (int)threadIdx.x; i < nb; i += (int)blockDim.x) {
-        const unsigned long long k = part[(long)m * nb + i];
-        best = k > best ? k : best;
+    for (int i0 = (int)threadIdx.x; i0 < nb; i0 += kGreedyThreads * kGreedyKeys) {
+        unsigned long long k[kGreedyKeys];
+#pragma unroll
+        for (int u = 0; u < kGreedyKeys; ++u) {
+            const int i = i0 + u * kGreedyThreads;
+            k[u] = keys[i < nb ? i : i0];  // past the end: a key already taken
+        }
+#pragma unroll
+        for (int u = 0; u < kGreedyKeys; ++u) best = k[u] > best ? k[u] : best;
     }
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
         const unsigned long long o = __shfl_xor(best, d);
         best = o > best ? o : best;
     }
-    __shared__ unsigned long long wbest[4];
+    __shared__ unsigned long long wbest[kGreedyThreads / 64];
     if ((threadIdx.x & 63) == 0) wbest[threadIdx.x >> 6] = best;
     __syncthreads();
     if (threadIdx.x == 0) {
-        for (int w = 1; w < (int)(blockDim.x >> 6); ++w) best = wbest[w] > best ? wbest[w] : best;
+#pragma unroll
+        for (int w = 1; w < kGreedyThreads / 64; ++w) best = wbest[w] > best ? wbest[w] : best;
         token[m] = greedy_index(best);
         if (value != nullptr) value[m] = greedy_value(best);
     }
@@ -758,7 +772,7 @@ __global__ __launch_bounds__(256) void greedy_reduce_kernel(const unsigned long 
 
 hipError_t launch_greedy_reduce(const unsigned long long* part, int nb, int m, int32_t* token, float* value,
                                 hipStream_t stream) {
-    hipLaunchKernelGGL(greedy_reduce_kernel, dim3(m), dim3(256), 0, stream, part, nb, token, value);
+    hipLaunchKernelGGL(greedy_reduce_kernel, dim3(m), dim3(kGreedyThreads), 0, stream, part, nb, token, value);
     return hipGetLastError();
 }
 
