@@ -903,6 +903,20 @@ __global__ __launch_bounds__(BN * 2) void gemm_kernel(const uint4* __restrict__ 
                 // the LDS table reads are issued together rather than waited for one by one
                 acc[i][j][0] = geglu2(OUT, slane & 15, acc[i][j][0], acc[i][j][1], gtab);
                 acc[i][j][2] = geglu2(OUT, slane & 15, acc[i][j][2], acc[i][j][3], gtab);
+                // sixteen table reads at a time, their results pinned here: left to itself the
+                // compiler finishes the values at their stores and keeps all 64 parts live
+                if (j == kNT - 1 && i % 4 == 3) {
+#pragma unroll
+                    for (int q = i - 3; q <= i; ++q)
+#pragma unroll
+                        for (int r = 0; r < kNT; ++r) {
+                            float h0 = acc[q][r][0], h2 = acc[q][r][2];
+                            asm volatile("" : "+v"(h0), "+v"(h2));
+                            acc[q][r][0] = h0;
+                            acc[q][r][2] = h2;
+                        }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
                 continue;
             }
             if constexpr (OUT == kOutGegluF32) {  // no memory reads: value and store together
