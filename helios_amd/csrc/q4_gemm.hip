@@ -50,6 +50,7 @@
 #include <type_traits>
 
 #include "q4_common.h"
+#include "q4_gemm_tile.h"
 #include "q4_kernels.h"
 
 namespace q4 {
@@ -60,26 +61,6 @@ constexpr int kNT = kWN / 16;         // 16x16 tiles per wave along N
 
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
 
-
-// The bias MFMA's A operand for one 16-row tile and one octet, as 64 lanes of 16 B:
-// lane (m = l%16, kq = l/16), element e -> group 8*octet + 2*kq + e/4, term e%4 in
-// {Xh, Xl, c Xh, c Xl} (c = -16, or 8 in the fp16 form).  Lane (m, kq) packs it from X
-// of row m for groups 2kq and 2kq + 1.
-template <int C = -16>
-__device__ __forceinline__ uint4 bias_a_operand(float x0, float x1) {
-    uint32_t w[4];
-    const float xs[2] = {x0, x1};
-#pragma unroll
-    for (int gi = 0; gi < 2; ++gi) {
-        const uint16_t xh = f32_to_bf16(xs[gi]);
-        const uint16_t xl = f32_to_bf16(xs[gi] - __uint_as_float((uint32_t)xh << 16));
-        const uint16_t nxh = f32_to_bf16((float)C * __uint_as_float((uint32_t)xh << 16));
-        const uint16_t nxl = f32_to_bf16((float)C * __uint_as_float((uint32_t)xl << 16));
-        w[2 * gi] = (uint32_t)xh | ((uint32_t)xl << 16);
-        w[2 * gi + 1] = (uint32_t)nxh | ((uint32_t)nxl << 16);
-    }
-    return make_uint4(w[0], w[1], w[2], w[3]);
-}
 
 // ---------------------------------------------------------------------------
 // X_g for the 256-row tile: bias A operands of every 16-row block and octet,
@@ -271,128 +252,6 @@ __global__ void scale_range_kernel(const uint2* __restrict__ sb, long records, i
         atomicMax(&out[0], emax);
         atomicMin(&out[1], emin);
         if (bad) atomicAdd(&out[2], bad);
-    }
-}
-
-// B operand of the bias MFMA from one scale/bias word pair: [b0 b0 s0 s0 b1 b1 s1 s1]
-__device__ __forceinline__ bf16x8 bias_operand(uint2 sbw) {
-    uint4 d;
-    d.x = __builtin_amdgcn_perm(sbw.x, sbw.x, 0x03020302u);  // b0 | b0 << 16
-    d.y = __builtin_amdgcn_perm(sbw.x, sbw.x, 0x01000100u);  // s0 | s0 << 16
-    d.z = __builtin_amdgcn_perm(sbw.y, sbw.y, 0x03020302u);
-    d.w = __builtin_amdgcn_perm(sbw.y, sbw.y, 0x01000100u);
-    return __builtin_bit_cast(bf16x8, d);
-}
-
-// Tile order: the hardware deals workgroup ids round-robin over the 8 XCDs; give
-// each XCD a contiguous run of tiles, and walk tiles in bands of two M tiles
-// (M fastest) so workgroups running together share x rows and weight tiles in L2.
-__device__ __forceinline__ void tile_of(int id, int nwg, int mtiles, int ntiles, int& mt, int& nt) {
-    constexpr int kXcds = 8;
-    int tile = id;
-    if (nwg % kXcds == 0) tile = (id % kXcds) * (nwg / kXcds) + id / kXcds;
-    constexpr int kBand = 2;
-    const int band = tile / (kBand * ntiles);
-    const int r = tile - band * kBand * ntiles;
-    const int bm = (mtiles - band * kBand) < kBand ? (mtiles - band * kBand) : kBand;
-    mt = band * kBand + r % bm;
-    nt = r / bm;
-}
-
-// t = x . A^T of a workgroup's BM rows into LDS (`ts`, [BM][rank] floats: the x ring's
-// first slot, BM x 128 bytes, so rank <= 32), each entry summed over its slices in
-// slice order; rows past the output read as zeros.  All of the workgroup's threads,
-// one barrier after.
-template <int BM>
-__device__ __forceinline__ void lora_stage_t(const LoraEpilogue& lo, float* ts, int row0, int m_rows, int nthr) {
-    const int q4s = lo.rank >> 2;  // float4s per row
-    for (int t = (int)threadIdx.x; t < BM * q4s; t += nthr) {
-        const int row = t / q4s, r = 4 * (t - row * q4s);
-        const int m = row0 + row;
-        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (m < m_rows) {
-            v = *reinterpret_cast<const float4*>(lo.part + (long)m * lo.rank + r);
-            for (int sl = 1; sl < lo.slices; ++sl) {
-                const float4 u = *reinterpret_cast<const float4*>(lo.part + ((long)sl * m_rows + m) * lo.rank + r);
-                v.x = v.x + u.x;
-                v.y = v.y + u.y;
-                v.z = v.z + u.z;
-                v.w = v.w + u.w;
-            }
-        }
-        *reinterpret_cast<float4*>(ts + row * lo.rank + r) = v;
-    }
-    __syncthreads();
-}
-
-// Eight fp32 values as bf16 high parts and the bf16 roundings of what is left
-// (v = hi + lo to about 2^-16 relative).
-__device__ __forceinline__ void split_bf16x8(const float4 a, const float4 b, bf16x8& hi, bf16x8& lo) {
-    const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        const __bf16 h = (__bf16)v[e];
-        hi[e] = h;
-        lo[e] = (__bf16)(v[e] - (float)h);
-    }
-}
-
-// The LoRA delta of a wave's output tiles and the combined store, in lora_up's
-// rounding steps (q4_lora.hip): d[m, n] = sum_r t[m, r] B[n, r] on the bf16 matrix
-// cores, t and B each split into bf16 high and low parts, d = th.bh + th.bl + tl.bh
-// (three 16x16x32 MFMAs per tile cover every rank up to 32; the dropped tl.bl term and
-// the parts' roundings leave d within about 2^-16 of the fp32 sum, far below the bf16
-// rounding of the delta that follows); then y = bf16(bf16(acc) + bf16(d * bf16(scale)))
-// in bf16, acc + d * scale in fp32.  Lane (row or column, kq) holds ranks 8kq..8kq+7;
-// columns past the output and ranks past the adapter's read zeros.
-template <bool F32, int kMT, int kNT>
-__device__ __forceinline__ void lora_store(const f32x4 (&acc)[kMT][kNT], const LoraEpilogue& lo, const float* ts,
-                                           void* y, int row0, int rb0, int m_rows, int n_rows, int lane) {
-#pragma clang fp contract(off)
-    const int col = lane & 15, kq = lane >> 4;
-    const int r0 = 8 * kq;
-    const float4 zero4 = make_float4(0.f, 0.f, 0.f, 0.f);
-    bf16x8 bh[kNT], bl[kNT];
-#pragma unroll
-    for (int j = 0; j < kNT; ++j) {
-        const int n = (rb0 + j) * 16 + col;
-        const bool ok = n < n_rows;
-        const float* bp = lo.b + (long)(ok ? n : 0) * lo.rank + r0;
-        const float4 b0 = ok && r0 < lo.rank ? *reinterpret_cast<const float4*>(bp) : zero4;
-        const float4 b1 = ok && r0 + 4 < lo.rank ? *reinterpret_cast<const float4*>(bp + 4) : zero4;
-        split_bf16x8(b0, b1, bh[j], bl[j]);
-    }
-    const float sc = F32 ? lo.scale : (float)(__bf16)lo.scale;
-    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int i = 0; i < kMT; ++i) {
-        const float* tp = ts + (16 * i + col) * lo.rank + r0;
-        const float4 t0 = r0 < lo.rank ? *reinterpret_cast<const float4*>(tp) : zero4;
-        const float4 t1 = r0 + 4 < lo.rank ? *reinterpret_cast<const float4*>(tp + 4) : zero4;
-        bf16x8 th, tl;
-        split_bf16x8(t0, t1, th, tl);
-#pragma unroll
-        for (int j = 0; j < kNT; ++j) {
-            f32x4 d = mfma16x16x32(th, bh[j], zero);
-            d = mfma16x16x32(th, bl[j], d);
-            d = mfma16x16x32(tl, bh[j], d);
-            const int n = (rb0 + j) * 16 + col;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int mr = row0 + 16 * i + 4 * kq + e;
-                if (mr < m_rows && n < n_rows) {
-                    const long o = (long)mr * n_rows + n;
-                    if constexpr (F32) {
-                        const float delta = d[e] * lo.scale;
-                        static_cast<float*>(y)[o] = acc[i][j][e] + delta;
-                    } else {
-                        const float base = (float)(__bf16)acc[i][j][e];
-                        const float delta = (float)(__bf16)(d[e] * sc);
-                        static_cast<uint16_t*>(y)[o] = f32_to_bf16(base + delta);
-                    }
-                }
-            }
-        }
     }
 }
 
@@ -1044,39 +903,50 @@ __global__ void split_geglu_kernel(const float* __restrict__ part, void* __restr
 
 }  // namespace
 
-// Tile shape and split of K.  For each tile shape (256, 128 or 64 rows x 256) and split
-// count (whole octets per split), the cost is
-//   rounds of workgroups x (groups per split x the step time + kRoundUs)
-//   + for a split: kSplitUs + the partial sums' bytes / kPartialBytesPerUs
-//   + for the 256-row tile: kPrePassUs (its X_g pre-pass launch),
-// and the cheapest wins.  The constants are fitted to every plan measured on the eight
-// prefill shapes (q, k, o, gate, down, the gate|up pair, the full-attention q and o) at
-// 14 row counts from 64 to 2048, every tile at every row count: the picks average 0.7%
-// and at worst 7.4% over the fastest plan of each case.  (The constants fitted to the
-// kernel with the pre-pass for every tile, the 64-row tile offered up to 128 rows,
-// give 3.7% and 26% on the same measurements.)
+// Tile shape and split of K.  For each tile and split count (whole octets per split) the
+// cost in us is
+//   rounds of workgroups x (a workgroup's time, body) x (1 + kFill x the rounds' fill)
+//   + for a split: kSplitUs + kPerSplitUs per split + the partial sums' bytes
+//   + for a pre-pass (the 256-row tile's X_g; x16 in its forms): kPrePassUs and x16's bytes,
+// and the cheapest wins.  The fill term is the clock and the memory shared by more
+// workgroups.  The constants are fitted (least squares of the logarithm) to every plan
+// within 1.5x of the best of its case, measured as forwards in a graph over rotated
+// weight copies on five shapes (qkv 8192x3840, o 3840x4096, down 3840x15360, k 2048x3840,
+// the gate|up pair 30720x3840) at eleven row counts from 40 to 1100, every tile with 1, 2,
+// 3, 4, 5 and 8 splits: the picks average 0.3% and at worst 6.2% over the fastest plan
+// of each case.  (The constants before, without the kpair tiles, chose up to 46% slower
+// than the best tile of their own at those sizes: the pair at 1100 rows 413 us against
+// 330 on the 64-row tile, and 282 on a kpair tile of 112 rows.)
 namespace {
 struct TileShape {
-    int bm, bn, per_cu;
-    double step_us;  // one 64-wide group step of a workgroup (fitted with the constants below)
-    int max_m;       // offered up to this many rows (0: any)
+    int bm, bn;
+    bool kpair;  // q4_gemm_kpair.hip
 };
-// The 64-row tile pads least and, unsplit, needs no scratch; it wins wherever it fills
-// the CUs with fewer K splits.  Best plan of each tile, measured: at 64 rows the
-// 128-row tile, half of it padding, is 10-26% behind (q 4096x3840 26.3 us vs 29.2, gate
-// 15360x3840 30.2 vs 36.1, the gate|up pair 41.7 vs 52.7); at 2048 rows k 2048x3840
-// runs 45.9 us on it unsplit against 57.7 on the 128-row tile split in two, and at 512
-// rows the full-attention q 8192x3840 46.5 vs 57.6.  Step times are fitted at one
-// workgroup per CU (the 64-row tile fits two, but each then runs at half the rate).
-constexpr TileShape kTileShapes[] = {{256, 256, 1, 1.8, 0}, {128, 256, 1, 1.1, 0}, {64, 256, 1, 0.65, 0}};
-constexpr double kRoundUs = 1.0;               // per round of workgroups: prologue, epilogue, ramp
-constexpr double kSplitUs = 4.0;               // a split's reduction launch
-constexpr double kPartialBytesPerUs = 4.0e6;   // partial sums written and read back
-constexpr double kPrePassUs = 3.0;             // the 256-row tile's group-sum pre-pass
+// The bf16 form on 64-row tiles is behind the kpair tiles in every case measured (at 64
+// rows qkv 16.7 us against 12.8, the pair 33.2 against 31.5; at 1100 rows 107 against 85
+// and 331 against 282) and is offered only to handles those cannot address; the 128-row
+// tile is ahead of them where it leaves no round short (the pair at 256 rows 74.5 against
+// 77.6).
+constexpr TileShape kTileShapes[] = {{256, 256, false}, {128, 256, false}, {64, 256, false}, {32, 256, true},
+                                     {48, 256, true},   {64, 256, true},   {80, 256, true},  {96, 256, true},
+                                     {112, 256, true}};
+constexpr double kFill = 0.372;
+constexpr double kSplitUs = 3.9, kPerSplitUs = 0.39;  // a split's reduction launch
+constexpr double kPartialBytesPerUs = 20.0e6;         // partial sums written and read back (mostly in the caches)
+constexpr double kPrePassUs = 3.0;                    // a pre-pass launch
+// a workgroup's time over `groups` groups, alone on its CU
+double body_us(const TileShape& ts, double step_scale, int groups) {
+    if (ts.kpair) {
+        const double mt = ts.bm / 16;
+        return groups / 4.0 * (0.688 + 0.243 * mt) + 0.09 + 0.765 * mt;
+    }
+    const double step = ts.bm == 256 ? 1.211 : ts.bm == 128 ? 0.773 : 0.46;
+    return groups * step * step_scale + 1.614 * (1.0 + ts.bm / 64.0);
+}
 // the fp16 form: its group step against the bf16 form's (gate 15360x3840 at 2048 rows,
 // the kernel alone, steady clock: 210-215 vs 218-223 us), and its pre-pass's extra
 // time per byte of x16 (12.3 us against the group-sum pre-pass's 5.0 for 15.7 MB)
-constexpr double kF16StepScale = 0.965;
+constexpr double kF16StepScale = 0.95;
 constexpr double kPrepBytesPerUs = 2.15e6;
 // one-pass 8-bit: its group step (over K, not 2K) against the 4-bit tile's of the
 // same height (8-bit gate 15360x3840 at 2048 rows with the pre-pass: 262 us on 256-row
@@ -1117,15 +987,17 @@ GemmPlan plan_gemm(int m, const Layout& l, size_t max_workspace) {
     // one-pass 8-bit: a two-plane handle whose low plane's group pairs line up with the
     // high plane's (an even number of groups per plane)
     const bool q8_ok = l.prepass_forms && l.k == 2 * l.kx && (l.g / 2) % 2 == 0 && l.kx / 64 <= kPrepMaxGroups;
+    const bool kp = kpair_fits(m, l);
     double best = -1.0;
     for (const TileShape& ts : kTileShapes) {
-        if (ts.max_m > 0 && m > ts.max_m) continue;
         const int bm = ts.bm, bn = ts.bn;
+        if (ts.kpair ? !kp : (bm == 64 && kp)) continue;
         const long tiles = (long)((m + bm - 1) / bm) * ((l.n + bn - 1) / bn);
         // form 0: the bf16 form; 1: the fp16 form (256-row tiles of handles whose scales
         // allow it); 2: one-pass 8-bit (128- and 256-row tiles)
         for (int form = 2; form >= 0; --form) {
-            if ((form == 1 && !(bm == 256 && l.f16 && l.prepass_forms)) || (form == 2 && !(bm >= 128 && q8_ok)))
+            if ((form == 1 && !(bm == 256 && l.f16 && l.prepass_forms)) || (form == 2 && !(bm >= 128 && q8_ok)) ||
+                (form != 0 && ts.kpair))
                 continue;
             const bool pre = form != 0;
             const int groups = form == 2 ? l.g / 2 : l.g;
@@ -1142,15 +1014,18 @@ GemmPlan plan_gemm(int m, const Layout& l, size_t max_workspace) {
                 const size_t part = s > 1 ? (size_t)s * m * l.n * 4 : 0;
                 if (part > kMaxPartialBytes) break;
                 if (xa + x16 + rexp + part > max_workspace) break;  // (more splits need more)
-                const double rounds = (double)((tiles * s + cus * ts.per_cu - 1) / (cus * ts.per_cu));
-                const double step = ts.step_us * (form == 1 ? kF16StepScale : form == 2 ? kQ8StepScale : 1.0);
-                const double t = rounds * (per * 8 * step + kRoundUs) +
-                                 (s > 1 ? kSplitUs + part / kPartialBytesPerUs : 0.0) +
+                const double wgs = (double)(tiles * s);
+                const double rounds = (double)((tiles * s + cus - 1) / cus);
+                const double scale = form == 1 ? kF16StepScale : form == 2 ? kQ8StepScale : 1.0;
+                const int gs = per * 8 < groups ? per * 8 : groups;
+                const double t = rounds * body_us(ts, scale, gs) * (1.0 + kFill * wgs / (rounds * cus)) +
+                                 (s > 1 ? kSplitUs + kPerSplitUs * s + part / kPartialBytesPerUs : 0.0) +
                                  ((bm == 256 || pre) ? kPrePassUs + x16 / kPrepBytesPerUs : 0.0);
                 if (best < 0.0 || t < best) {
                     best = t;
                     p.bm = bm;
                     p.bn = bn;
+                    p.kpair = ts.kpair;
                     p.splits = s;
                     p.g_split = per * 8;
                     p.part_bytes = part;
@@ -1230,7 +1105,11 @@ hipError_t launch_gemm(const uint4* tiles, const uint2* sb, const uint16_t* x, v
         STRIDE, n_out, gelu_table, lo, rowexp, s_pow, lo_pairs
 #define Q4_GEMM_LAUNCH(MODE, YPTR, STRIDE)                                                                       \
     do {                                                                                                         \
-        if (plan.bm == 64)                                                                                       \
+        if (plan.kpair) {                                                                                        \
+            const hipError_t ek = launch_kpair(tiles, sb, x, YPTR, m, MODE, n_out, l, plan, STRIDE, gelu_table,  \
+                                               lo, stream);                                                      \
+            if (ek != hipSuccess) return ek;                                                                     \
+        } else if (plan.bm == 64)                                                                                       \
             hipLaunchKernelGGL((gemm_kernel<MODE, 64, 256>), grid, block, 0, stream, Q4_GEMM_ARGS(YPTR, STRIDE));  \
         else if (plan.bm == 256 && plan.f16)                                                                     \
             hipLaunchKernelGGL((gemm_kernel<MODE, 256, 256, 1>), grid, block, 0, stream,                         \

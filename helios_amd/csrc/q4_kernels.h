@@ -7,6 +7,8 @@
 
 namespace q4 {
 
+struct LoraEpilogue;
+
 // Weight records: one per (16-row block, group pair), [row block][pair], 1152 bytes
 // each: the 1 KiB tile of tiled words (uint4 per lane) and then the block's 16 scale/
 // bias words for the pair (uint2 per row), so a kernel streaming a row block reads one
@@ -24,6 +26,8 @@ constexpr int kRecU2 = kRecBytes / 8;
 __host__ __device__ inline uint32_t sb_span(int n) {
     return n > 0 ? (uint32_t)n * (uint32_t)kRecBytes - (uint32_t)kRecSbBytes : 0u;
 }
+
+constexpr size_t kMaxRecBytes = (size_t)1 << 31;  // a buffer resource's
 
 struct Layout {
     int n = 0;   // output features
@@ -138,13 +142,14 @@ void set_f16_form(Layout& l, const int range[3]);
 // `workspace_bytes`; gemm_workspace_bytes(m, l) is what the unconstrained plan
 // needs, and with that much the launch runs the unconstrained plan.
 struct GemmPlan {
-    int bm = 256;            // output tile rows: 256, 128 or 64
+    int bm = 256;            // output tile rows
     int bn = 256;            // output tile columns
     int splits = 1;          // workgroups along K per output tile
     int g_split = 0;         // groups per split (whole octets)
     size_t xaug_bytes = 0;   // group sums of x (256-row tiles)
     size_t part_bytes = 0;   // splits x M x N fp32 partial sums (0 when unsplit)
     bool f16 = false;        // fp16 form (256-row tiles of a handle whose scales allow it)
+    bool kpair = false;      // q4_gemm_kpair.hip: tiles of 32, 48, .. 112 rows x 256
     bool q8 = false;         // one-pass 8-bit (128-row tiles of a two-plane handle)
     size_t x16_bytes = 0;    // fp16 and one-pass 8-bit forms: x scaled per row, as fp16 [M, kx]
     size_t rowexp_bytes = 0; // their rows' powers of two
@@ -162,6 +167,19 @@ int device_cus();
 hipError_t launch_gemm(const uint4* tiles, const uint2* sb, const uint16_t* x, void* y, int m, int out_mode,
                        int n_out, const Layout& l, void* workspace, size_t workspace_bytes,
                        const uint16_t* gelu_table, hipStream_t stream, const LoraEpilogue* lora = nullptr);
+// One launch of a kpair plan (q4_gemm_kpair.hip): y in out_mode (a mode of the GEMM), or
+// the partial planes of a split; lora only in the LoRA modes.
+hipError_t launch_kpair(const uint4* tiles, const uint2* sb, const uint16_t* x, void* y, int m, int out_mode, int n_out,
+                        const Layout& l, const GemmPlan& plan, long split_stride, const uint16_t* gelu_table,
+                        const LoraEpilogue& lora, hipStream_t stream);
+// Whether its 32-bit offsets reach everything: a tile's rows past x and row blocks past
+// the records (offsets that read as zero must not wrap), and a tile's rows of y.
+constexpr int kKpairMaxRows = 112;  // rows of the largest kpair tile
+inline bool kpair_fits(int m, const Layout& l) {
+    const size_t wrap = (size_t)1 << 32;
+    return ((size_t)m + kKpairMaxRows) * l.kx * 2 < wrap && l.rec_bytes() + (size_t)16 * l.gp * kRecBytes < wrap &&
+           l.rec_bytes() <= kMaxRecBytes && (size_t)kKpairMaxRows * l.n * 4 < kMaxRecBytes;
+}
 // Whether launch_gemm can add a LoRA delta of this rank in its epilogue for m rows
 // within `workspace_bytes` (an unsplit plan; rank a multiple of 4 up to 32).
 bool gemm_lora_epilogue(int m, const Layout& l, int rank, size_t workspace_bytes);
@@ -188,20 +206,21 @@ hipError_t launch_lora(const uint16_t* x, const float* a, const uint16_t* a_hi, 
 hipError_t launch_lora_down(const uint16_t* x, const uint16_t* a_hi, const uint16_t* a_lo, float* part, int m,
                             int k, int rank, hipStream_t stream);
 
-// Forward path choice (automatic mode): the decode kernels below kGemmMinRows rows,
+// Forward path choice (automatic mode): the decode kernels up to 16 rows (one slab),
 // and beyond that while 16-row slabs x N x K stays at most kDecodeMaxSlabWork (K' = 2K
 // for two-plane 8-bit handles).  The decode kernels' cost grows by one pass over the
-// weights per 16-row slab (~0.24 us per million weights); the GEMM's starts at ~14 us
+// weights per 16-row slab (~0.24 us per million weights); the GEMM's starts at ~10 us
 // (launch, tile prologue and epilogue, split-K reduction) and grows slowly at these
-// sizes.  Measured as whole forwards (graph replays, each path pinned) on nine shapes
-// (q, k, o, the fused qkv, gate, down, the gate|up pair, the full-attention o and k)
-// at 32-256 rows: with any bound from 5e7 to 6e7 the choice is within 3% of the faster
-// path everywhere (q 4096x3840: decode to 48 rows, 15.3 vs 16.3 us; GEMM from 56,
-// 16.9 vs 18.3; the fused qkv 8192x3840 at 32 rows on the GEMM, 13.8 vs 19.9).
-constexpr int kGemmMinRows = 32;
-constexpr double kDecodeMaxSlabWork = 5.5e7;
-// The slab bound was fitted on the Gemma shapes at 32-256 rows (the full-attention k,
-// 512 x 3840, stays on decode to 448 rows); beyond 64 slabs the GEMM takes any shape.
+// sizes.  Measured as whole forwards (graph replays over rotated weight copies, each
+// path pinned) on eight shapes at 8-400 rows, decode / GEMM in us:
+//   up to the bound: o 3840x4096 at 17 rows 9.1 / 10.9, at 32 11.5 / 11.4; k 2048x3840 at
+//     64 11.0 / 11.8; the full-attention k 512x3840 at 256 10.8 / 11.8;
+//   past it: q 4096x3840 at 40 13.9 / 12.8; k at 96 14.9 / 12.9; qkv 8192x3840 at 17
+//     15.4 / 10.3; the gate|up pair at 17 38.5 / 23.9; down at 17 29.9 / 17.6.
+// (Up to 16 rows decode is ahead or within 15%: qkv at 16 11.4 / 10.3, the pair 21.7 / 24.1.)
+constexpr int kGemmMinRows = 17;
+constexpr double kDecodeMaxSlabWork = 3.5e7;
+// Beyond 64 slabs the GEMM takes any shape.
 constexpr long kDecodeMaxRows = 1024;
 inline bool use_decode(long rows, const Layout& l, int gemm_min_rows) {
     if (gemm_min_rows > 0) return rows < gemm_min_rows;
