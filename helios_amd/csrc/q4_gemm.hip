@@ -932,7 +932,10 @@ constexpr TileShape kTileShapes[] = {{256, 256, false}, {128, 256, false}, {64, 
                                      {112, 256, true}};
 constexpr double kFill = 0.372;
 constexpr double kSplitUs = 3.9, kPerSplitUs = 0.39;  // a split's reduction launch
-constexpr double kPartialBytesPerUs = 20.0e6;         // partial sums written and read back (mostly in the caches)
+constexpr double kPartialBytesPerUs = 20.0e6;         // partial sums written and read back, mostly in the caches
+// and past what those take (the 8-bit pair at 700 rows split in two, 172 MB: its reduction
+// 35 us, where the cached rate says 9)
+constexpr double kPartialCached = 32.0e6, kPartialFarBytesPerUs = 6.7e6;
 constexpr double kPrePassUs = 3.0;                    // a pre-pass launch
 // a workgroup's time over `groups` groups, alone on its CU
 double body_us(const TileShape& ts, double step_scale, int groups) {
@@ -1020,6 +1023,7 @@ GemmPlan plan_gemm(int m, const Layout& l, size_t max_workspace) {
                 const int gs = per * 8 < groups ? per * 8 : groups;
                 const double t = rounds * body_us(ts, scale, gs) * (1.0 + kFill * wgs / (rounds * cus)) +
                                  (s > 1 ? kSplitUs + kPerSplitUs * s + part / kPartialBytesPerUs : 0.0) +
+                                 (part > kPartialCached ? (part - kPartialCached) / kPartialFarBytesPerUs : 0.0) +
                                  ((bm == 256 || pre) ? kPrePassUs + x16 / kPrepBytesPerUs : 0.0);
                 if (best < 0.0 || t < best) {
                     best = t;
