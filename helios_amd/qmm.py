@@ -217,16 +217,19 @@ def gemm_min_rows(rows: int):
         set_gemm_min_rows(prev)
 
 
-def _stream_ptr(stream):
+def _stream_ptr(stream) -> int:
+    """The raw stream (default: torch's current one on the current device).  Read without
+    building a torch Stream object, which costs about as much as a launch; plain integers
+    here and in _dev_ptr: ctypes converts them to the declared void pointers itself."""
     import torch
 
     if stream is None:
-        stream = torch.cuda.current_stream()
-    return ctypes.c_void_p(stream.cuda_stream)
+        return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+    return stream.cuda_stream
 
 
-def _dev_ptr(t) -> ctypes.c_void_p:
-    return ctypes.c_void_p(t.data_ptr())
+def _dev_ptr(t) -> int:
+    return t.data_ptr()
 
 
 def _check_spec(group_size: int, bits: int, mode: str, transpose: bool = True) -> None:
@@ -280,15 +283,17 @@ def _run_forward(fn, handle, lib, x, in_features: int, out_features: int, out=No
         raise Gemma4Error(Status.INVALID_ARGUMENT, "x must be bfloat16")
     if x.shape[-1] != in_features:
         raise Gemma4Error(Status.INVALID_ARGUMENT, f"x last dim {x.shape[-1]} != in_features {in_features}")
-    lead = tuple(x.shape[:-1])
-    x2 = x.reshape(-1, in_features).contiguous()
+    lead = x.shape[:-1]
+    x2 = x if x.dim() == 2 and x.is_contiguous() else x.reshape(-1, in_features).contiguous()
     rows = x2.shape[0]
     if out is None:
-        out = torch.empty(lead + (out_features,), dtype=out_dtype, device=x.device)
-    elif out.dtype != out_dtype or tuple(out.shape) != lead + (out_features,) or not out.is_contiguous():
+        out = torch.empty((*lead, out_features), dtype=out_dtype, device=x.device)
+    elif out.dtype != out_dtype or tuple(out.shape) != (*lead, out_features) or not out.is_contiguous():
         raise Gemma4Error(Status.INVALID_ARGUMENT, "out has the wrong dtype, shape or layout")
-    code = DTYPE_F32 if out_dtype == torch.float32 else DTYPE_BF16
-    check(fn(handle, _stream_ptr(stream), _dev_ptr(x2), rows, _dev_ptr(out), code), lib)
+    status = fn(handle, _stream_ptr(stream), x2.data_ptr(), rows, out.data_ptr(),
+                DTYPE_F32 if out_dtype == torch.float32 else DTYPE_BF16)
+    if status != 0:
+        check(status, lib)
     return out
 
 
