@@ -1,4 +1,4 @@
-// Decode-shape affine-Q4 matmul on gfx950: y[M,N] = x[M,K] . W^T for M < 32 (and
+// Decode-shape affine-Q4 matmul on gfx950: y[M,N] = x[M,K] . W^T for M <= 16 (and
 // beyond, for weights small enough that slabs beat the GEMM's fixed costs), in
 // 16-row slabs (one launch; slab = blockIdx.y).
 //

@@ -1,4 +1,5 @@
-// Prefill-shape affine-Q4 matmul on gfx950: y[M,N] = x[M,K] . W^T for large M.
+// Prefill-shape affine-Q4 matmul on gfx950: y[M,N] = x[M,K] . W^T for large M, and the
+// plan and launch of every GEMM (tiles of 32 to 112 rows: q4_gemm_kpair.hip).
 //
 // Exact factored form on the matrix cores (q4_common.h):
 //   y = sum_g 16*s_g * P_g + (b_g - 16*s_g) * X_g,   P_g = sum_{k in g} x*(1 + q/16)
