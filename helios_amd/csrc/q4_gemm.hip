@@ -913,9 +913,9 @@ __global__ void split_geglu_kernel(const float* __restrict__ part, void* __restr
 // workgroups.  The constants are fitted (least squares of the logarithm) to every plan
 // within 1.5x of the best of its case, measured as forwards in a graph over rotated
 // weight copies on five shapes (qkv 8192x3840, o 3840x4096, down 3840x15360, k 2048x3840,
-// the gate|up pair 30720x3840) at eleven row counts from 40 to 1100, every tile with 1, 2,
-// 3, 4, 5 and 8 splits: the picks average 0.3% and at worst 6.2% over the fastest plan
-// of each case.  (The constants before, without the kpair tiles, chose up to 46% slower
+// the gate|up pair 30720x3840) at fourteen row counts from 20 to 1600, every tile with 1,
+// 2, 3, 4, 5 and 8 splits: the picks average 0.2% and at worst 4.7% over the fastest of
+// those plans.  (The constants before, without the kpair tiles, chose up to 46% slower
 // than the best tile of their own at those sizes: the pair at 1100 rows 413 us against
 // 330 on the 64-row tile, and 282 on a kpair tile of 112 rows.)
 namespace {
@@ -931,21 +931,21 @@ struct TileShape {
 constexpr TileShape kTileShapes[] = {{256, 256, false}, {128, 256, false}, {64, 256, false}, {32, 256, true},
                                      {48, 256, true},   {64, 256, true},   {80, 256, true},  {96, 256, true},
                                      {112, 256, true}};
-constexpr double kFill = 0.372;
-constexpr double kSplitUs = 3.9, kPerSplitUs = 0.39;  // a split's reduction launch
-constexpr double kPartialBytesPerUs = 20.0e6;         // partial sums written and read back, mostly in the caches
+constexpr double kFill = 0.426;
+constexpr double kSplitUs = 3.8, kPerSplitUs = 0.38;  // a split's reduction launch
+constexpr double kPartialBytesPerUs = 17.0e6;         // partial sums written and read back, mostly in the caches
 // and past what those take (the 8-bit pair at 700 rows split in two, 172 MB: its reduction
-// 35 us, where the cached rate says 9)
-constexpr double kPartialCached = 32.0e6, kPartialFarBytesPerUs = 6.7e6;
+// 35 us, where the cached rate says 10)
+constexpr double kPartialCached = 64.0e6, kPartialFarBytesPerUs = 6.7e6;
 constexpr double kPrePassUs = 3.0;                    // a pre-pass launch
 // a workgroup's time over `groups` groups, alone on its CU
 double body_us(const TileShape& ts, double step_scale, int groups) {
     if (ts.kpair) {
         const double mt = ts.bm / 16;
-        return groups / 4.0 * (0.688 + 0.243 * mt) + 0.09 + 0.765 * mt;
+        return groups / 4.0 * (0.693 + 0.261 * mt) + 0.737 * mt;
     }
-    const double step = ts.bm == 256 ? 1.211 : ts.bm == 128 ? 0.773 : 0.46;
-    return groups * step * step_scale + 1.614 * (1.0 + ts.bm / 64.0);
+    const double step = ts.bm == 256 ? 1.202 : ts.bm == 128 ? 0.766 : 0.46;
+    return groups * step * step_scale + 1.464 * (1.0 + ts.bm / 64.0);
 }
 // the fp16 form: its group step against the bf16 form's (gate 15360x3840 at 2048 rows,
 // the kernel alone, steady clock: 210-215 vs 218-223 us), and its pre-pass's extra
