@@ -220,12 +220,24 @@ hipError_t launch_lora_down(const uint16_t* x, const uint16_t* a_hi, const uint1
 // (Up to 16 rows decode is ahead or within 15%: qkv at 16 11.4 / 10.3, the pair 21.7 / 24.1.)
 constexpr int kGemmMinRows = 17;
 constexpr double kDecodeMaxSlabWork = 3.5e7;
+// From 9 rows a two-plane 8-bit handle's x' no longer fits the decode kernels' LDS beside
+// its steps, and with enough weights the GEMM is ahead there, too (decode / GEMM, us, at
+// 9, 12 and 16 rows): gate 27.8 / 23.6, 32.2 / 23.8, 38.0 / 23.9; the pair 52.9 / 38.8,
+// 61.7 / 39.0, 73.4 / 40.1; down 27.4 / 26.1, 32.4 / 26.0, 38.3 / 26.2; from 12 rows with
+// fewer: qkv 8192x3840 15.3 / 14.9, 17.6 / 15.0, 20.5 / 15.0; the full-attention o
+// 3840x8192 14.9 / 17.2, 17.2 / 17.2, 19.6 / 17.3; not o 3840x4096 (11.4 / 14.0 at 16).
+constexpr int kTwoPlaneRows[2] = {9, 12};
+constexpr double kTwoPlaneWork[2] = {1.0e8, 6.0e7};  // N x K' from that many rows on
 // Beyond 64 slabs the GEMM takes any shape.
 constexpr long kDecodeMaxRows = 1024;
 inline bool use_decode(long rows, const Layout& l, int gemm_min_rows) {
     if (gemm_min_rows > 0) return rows < gemm_min_rows;
-    return rows < kGemmMinRows ||
-           (rows <= kDecodeMaxRows && (double)((rows + 15) / 16) * (double)l.n * (double)l.k <= kDecodeMaxSlabWork);
+    if (rows < kGemmMinRows) {
+        if (l.kx == l.k || rows < kTwoPlaneRows[0]) return true;
+        return (double)l.n * (double)l.k < kTwoPlaneWork[rows < kTwoPlaneRows[1] ? 0 : 1];
+    }
+    return rows <= kDecodeMaxRows &&
+           (double)((rows + 15) / 16) * (double)l.n * (double)l.k <= kDecodeMaxSlabWork;
 }
 
 }  // namespace q4

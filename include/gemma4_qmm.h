@@ -125,7 +125,8 @@ Gemma4Status gemma4_qmm_get_last_error(char* buffer, size_t buffer_len);
  *     ceil(rows / 16) * N * K <= 3.5e7 (K' = 2K for 8-bit handles), the GEMM
  *     otherwise: for the Gemma 4 shapes the decode kernels are ahead of the GEMM's
  *     fixed costs up to 32 rows for 4096x3840, 64 for 2048x3840, 272 for 512x3840,
- *     and up to 16 rows for 8192x3840 and the MLP projections.
+ *     and up to 16 rows for 8192x3840 and the MLP projections.  8-bit handles go
+ *     to the GEMM from 9 rows with N * K' >= 1e8 and from 12 with N * K' >= 6e7.
  *   r > 0: the GEMM from r rows on, the decode kernels below.
  * Both paths meet the same accuracy contract; they sum in different orders, so the
  * last bits of some outputs differ between them.  Returns the previous setting.
