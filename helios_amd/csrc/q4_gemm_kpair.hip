@@ -164,12 +164,12 @@ __global__ __launch_bounds__(512) void kpair_kernel(const KpairArgs a) {
     // Step s (groups 4 s .. 4 s + 3): (0) the A operands of step s - 1's bias term, into
     // the slot of its parity (last read in step s - 2, a barrier ago); (1) wait until the
     // wave's x of this step, issued during step s - 1, has landed, leaving in flight the
-    // words issued after it; (2) barrier: everyone's x and operands are in LDS and
+    // ten loads issued after it; (2) barrier: everyone's x and operands are in LDS and
     // everyone is done with the x slot refilled next; (3) step s - 1's bias term; (4)
     // multiply, with the next step's loads spread through the products: x, then the words
     // of the wave's next pair in place once this pair's are expanded, then this step's
     // scale/bias words.  Every step issues the same loads (past the end they read zeros),
-    // so the count is fixed.
+    // so the count is fixed; the first step's x was waited for before the loop.
     auto step = [&](int s, auto odd_, const uint4* xs, uint4* xs2, PairWords& w) {
         constexpr bool kOdd = decltype(odd_)::value;
         if (s > s_begin) write_xa(!kOdd);
@@ -261,6 +261,9 @@ __global__ __launch_bounds__(512) void kpair_kernel(const KpairArgs a) {
     for (int u = 0; u < kMT; ++u) dma_x(s_begin, u, g_x0);
 #pragma unroll
     for (int j = 0; j < 4; ++j) load_w(s_begin, j, w);
+    // only the words' eight loads follow the first step's x (no scale/bias words ahead of
+    // it), so a step's own wait would leave the wave's last two x loads in flight
+    wait_vm<8>();
     for (int s = s_begin; s < s_end; s += 2) {
         step(s, std::integral_constant<bool, false>{}, g_x0, g_x1, w);
         if (s + 1 < s_end) step(s + 1, std::integral_constant<bool, true>{}, g_x1, g_x0, w);

@@ -41,6 +41,11 @@ def gemm_asm():
     return hbuild.device_asm("q4_gemm.hip")
 
 
+@pytest.fixture(scope="module")
+def kpair_asm():
+    return hbuild.device_asm("q4_gemm_kpair.hip")
+
+
 def test_lds_dma_sgpr_hazards_covered(gemm_asm):
     kernels = list(_kernels(gemm_asm))
     # bf16 / fp32 outputs, bf16 / fp32 GeGLU pairs, bf16 / fp32 outputs with a LoRA
@@ -85,6 +90,77 @@ def test_no_spills_and_lds_budget(gemm_asm):
             small += 1
             assert int(m.group(1)) <= 80 * 1024 and int(m.group(3)) <= 128, m.group(2)
     assert small == 6
+
+
+# --------------------------------------------------------------- LDS DMAs and barriers
+
+_COUNTED = re.compile(r"(buffer|global|flat|scratch)_(load|store|atomic)")
+
+
+def _blocks(asm: str, kernel: str):
+    """The kernel's code as basic blocks: [(instructions, successors)], the entry first."""
+    m = re.search(rf"\n(\S*{kernel}\S*):[^\n]*\n", asm)
+    body = asm[m.end():asm.index(".section", m.end())]
+    blocks, names = [[]], {}
+    for line in body.splitlines():
+        line = line.split(";")[0].strip()
+        label = re.match(r"(\.LBB\w+):$", line)
+        if label:
+            if blocks[-1]:
+                blocks.append([])
+            names[label.group(1)] = len(blocks) - 1
+        elif line and not line.startswith((".", "#")):
+            blocks[-1].append(line)
+            if line.startswith(("s_branch", "s_cbranch", "s_endpgm")):
+                blocks.append([])
+    out = []
+    for i, ins in enumerate(blocks):
+        last = ins[-1] if ins else ""
+        nxt = [names[last.split()[1]]] if last.startswith(("s_branch", "s_cbranch")) else []
+        if not last.startswith(("s_branch", "s_endpgm")) and i + 1 < len(blocks):
+            nxt.append(i + 1)
+        out.append((ins, nxt))
+    return out
+
+
+def _dmas_in_flight_at_barriers(asm: str, kernel: str):
+    """Barriers that some path reaches with an LDS DMA of the wave still in flight, as
+    (the barrier's text with its block's last instructions, loads issued after the DMA).
+    Memory operations return in order, so a DMA followed by n of them has landed at a
+    wait for vmcnt <= n; per block the worst path (the fewest operations after a DMA)."""
+    blocks = _blocks(asm, kernel)
+    state, work, bad, dmas = {0: None}, [0], {}, 0
+    while work:
+        b = work.pop()
+        after = state[b]  # operations after the newest DMA in flight; None: none in flight
+        for i, ins in enumerate(blocks[b][0]):
+            if _COUNTED.match(ins):
+                if re.search(r"\blds\b", ins):
+                    after, dmas = 0, dmas + 1
+                elif after is not None:
+                    after = min(after + 1, 64)
+            elif ins.startswith("s_waitcnt"):
+                n = re.search(r"vmcnt\((\d+)\)", ins)
+                if n and after is not None and int(n.group(1)) <= after:
+                    after = None
+            elif ins.startswith("s_barrier") and after is not None:
+                bad[(b, i)] = after
+        for n in blocks[b][1]:
+            old = state.get(n, "new")
+            new = after if old in ("new", None) else old if after is None else min(old, after)
+            if old == "new" or new != old:
+                state[n] = new
+                work.append(n)
+    assert dmas > 0, kernel
+    return bad
+
+
+@pytest.mark.parametrize("kmt", [2, 3, 4, 5, 6, 7])
+def test_kpair_x_has_landed_at_every_barrier(kpair_asm, kmt):
+    """Waves of the kpair GEMM read x rows that other waves' DMAs bring, so every DMA a
+    wave issued has landed when it reaches the next barrier.  The waits count the loads
+    issued after the DMAs: eight before the first step, ten in every later one."""
+    assert _dmas_in_flight_at_barriers(kpair_asm, f"kpair_kernelILi{kmt}E") == {}
 
 
 def _kernel_meta(asm: str):
