@@ -714,13 +714,13 @@ bool limb_rows_preferred(const Layout& l, int m) {
     // 8192x3840 6.8 against 7.3 us, o 3840x4096 5.2 against 5.4, q 5.2 against 5.4, k
     // 2048x3840 4.9 against 5.0; 1024-wide K even; o of K = 8192 8.3 against 7.8) and
     // at 3 rows from 512 row blocks (qkv 6.8 against 7.1; q 5.3 against 5.2).  From 5
-    // rows those lose (qkv 8.2 against 7.6-7.9 us, o 6.9 against 5.7).  Two-plane
-    // 8-bit handles gain at 3-4 rows from 512 row blocks (qkv 13.3 -> 11.2 us at 3 rows,
-    // 12.0 -> 11.3 at 4; gate 19.0 -> 16.8, 17.2 -> 16.1; the gate|up pair 28.3 -> 26.0,
-    // 28.0 -> 25.8), narrower ones lose there (o 7.7 against 8.5), and from 5 rows they are
-    // within 5% either way.
+    // rows those lose (qkv 8.2 against 7.6-7.9 us, o 6.9 against 5.7).  Not two-plane
+    // 8-bit handles: from 3 rows they take x as it is on the bf16 kernels, and 20 bits
+    // under a group's largest value would keep less of it (faster all the same where
+    // there are 512 row blocks or more: qkv at 3 rows 11.2 us against 13.3, the gate|up
+    // pair 26.0 against 28.3).
     const int cus = device_cus();
-    if (l.kx != l.k) return m <= 4 && l.nb >= 2 * cus;
+    if (l.kx != l.k) return false;
     if (l.nb >= 3 * cus) return true;
     return l.gp <= 32 && ((m == 4 && l.nb >= 128) || (m == 3 && l.nb >= 2 * cus));
 }

@@ -1,5 +1,5 @@
-"""8-bit handles at the row counts where their path changes: 3 and 4 rows on wide outputs
-(the int8 kernels from 512 row blocks, the bf16 ones below) and 8 to 17 rows around the
+"""8-bit handles at the row counts where their path changes: 2 to 5 rows (the int8 kernels
+up to 2, the bf16 ones from 3) and 8 to 17 rows around the
 GEMM's first (9 rows from N x 2K = 1e8, 12 from 6e7).  Every automatic result against the oracle and
 against both pinned paths: fp32 outputs within GEMM_REL of the RMS (the kernels' sums are
 exact products in fp32, in different orders)."""
@@ -41,3 +41,36 @@ def test_q8_row_rules(gpu_lib, n, k, rows):
         for other in (gm, dc):
             assert float((y32 - other).abs().max()) <= GEMM_REL * rms, m
     lin.close()
+
+
+@pytest.mark.parametrize("n", [8192, 65536 + 16])
+@pytest.mark.parametrize("m", [3, 4])
+def test_q8_small_x_beside_large(gpu_lib, n, m):
+    """x is taken as it is at 3-4 rows of an 8-bit handle, whatever else its group holds:
+    rows of one value 1 and 63 of 0.75 x 2^-21 a group (below what 20 bits under the
+    group's largest keep), and rows of bf16 subnormals only.  The large value's weight is
+    exactly 0, so the result is the small values'.  fp32 sums of the factored form
+    (weights as 16 s (1 + q/16) on two planes): each group's terms total at most 512 s
+    sum |x|, and eight roundings of 2^-24 of that bound the error."""
+    import torch
+
+    k = 256
+    rng = np.random.default_rng(n + m)
+    codes = rng.integers(192, 256, (n, k)).astype(np.uint8)
+    codes[:, ::64] = 128
+    w = np.ascontiguousarray(codes).view(np.uint32)
+    sf = A.round_to_bf16((rng.random((n, k // 64)) * 0.01 + 0.002).astype(np.float32))
+    tri = (w, A.f32_to_bf16_bits(sf), A.f32_to_bf16_bits(-128.0 * sf))
+    xf = np.full((m, k), 0.75 * 2.0 ** -21, np.float32)
+    xf[:, ::64] = 1.0
+    x = A.f32_to_bf16_bits(xf)
+    x[m - 1] = rng.integers(0x20, 0x80, k)  # subnormals only
+    lin = gpu_lib.QuantizedLinear(*dev_triple(*tri), bits=8)
+    y = lin.forward(dev_x(x), out_dtype=torch.float32).cpu().numpy().astype(np.float64)
+    lin.close()
+    want = C.qmm_f64(x, *tri, bits=8)
+    xs = np.abs(A.bf16_bits_to_f32(x).astype(np.float64)).reshape(m, k // 64, 64).sum(axis=2)
+    bound = 8 * 2.0 ** -24 * 512 * xs @ sf.astype(np.float64).T
+    assert (want > 4 * bound).all()
+    worst = (np.abs(y - want) / bound).max(axis=1)
+    assert (worst <= 1).all(), worst
