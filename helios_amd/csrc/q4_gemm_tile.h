@@ -78,57 +78,50 @@ __device__ __forceinline__ void lora_stage_t(const LoraEpilogue& lo, float* ts, 
     __syncthreads();
 }
 
-// Eight fp32 values as bf16 high parts and the bf16 roundings of what is left
-// (v = hi + lo to about 2^-16 relative).
-__device__ __forceinline__ void split_bf16x8(const float4 a, const float4 b, bf16x8& hi, bf16x8& lo) {
-    const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        const __bf16 h = (__bf16)v[e];
-        hi[e] = h;
-        lo[e] = (__bf16)(v[e] - (float)h);
-    }
-}
-
 // The LoRA delta of a wave's output tiles and the combined store, in lora_up's
-// rounding steps (q4_lora.hip): d[m, n] = sum_r t[m, r] B[n, r] on the bf16 matrix
-// cores, t and B each split into bf16 high and low parts, d = th.bh + th.bl + tl.bh
-// (three 16x16x32 MFMAs per tile cover every rank up to 32; the dropped tl.bl term and
-// the parts' roundings leave d within about 2^-16 of the fp32 sum, far below the bf16
-// rounding of the delta that follows); then y = bf16(bf16(acc) + bf16(d * bf16(scale)))
-// in bf16, acc + d * scale in fp32.  Lane (row or column, kq) holds ranks 8kq..8kq+7;
-// columns past the output and ranks past the adapter's read zeros.
+// rounding steps (q4_lora.hip): d[m, n] = sum_r t[m, r] B[n, r] in fp32 on the matrix
+// cores (16x16x4), as close to the exact sum as lora_up's, which takes the delta of plans
+// that split K; then y = bf16(bf16(acc) + bf16(d * bf16(scale))) in bf16, acc + d * scale
+// in fp32.  Lane (row or column, kq) holds ranks 4 kq .. 4 kq + 3 of each 16, one float4
+// for four products; columns past the output and ranks past the adapter's are zeros.
+// (t and B in two bf16 parts, three 16x16x32 products, left an fp32 output's delta
+// 74 x 2^-24 off, so 3; the time is the same on kpair tiles, q|k|v|o of 1100 rows at rank
+// 16 202 us, and 240 / 242 us for gate at 2048 rows and rank 16, 255 / 263 at rank 32.)
 template <bool F32, int kMT, int kNT>
 __device__ __forceinline__ void lora_store(const f32x4 (&acc)[kMT][kNT], const LoraEpilogue& lo, const float* ts,
                                            void* y, int row0, int rb0, int m_rows, int n_rows, int lane) {
 #pragma clang fp contract(off)
     const int col = lane & 15, kq = lane >> 4;
-    const int r0 = 8 * kq;
+    const int r0 = 4 * kq, r1 = 16 + 4 * kq;
     const float4 zero4 = make_float4(0.f, 0.f, 0.f, 0.f);
-    bf16x8 bh[kNT], bl[kNT];
+    float4 b0[kNT], b1[kNT];
 #pragma unroll
     for (int j = 0; j < kNT; ++j) {
         const int n = (rb0 + j) * 16 + col;
         const bool ok = n < n_rows;
-        const float* bp = lo.b + (long)(ok ? n : 0) * lo.rank + r0;
-        const float4 b0 = ok && r0 < lo.rank ? *reinterpret_cast<const float4*>(bp) : zero4;
-        const float4 b1 = ok && r0 + 4 < lo.rank ? *reinterpret_cast<const float4*>(bp + 4) : zero4;
-        split_bf16x8(b0, b1, bh[j], bl[j]);
+        const float* bp = lo.b + (long)(ok ? n : 0) * lo.rank;
+        b0[j] = ok && r0 < lo.rank ? *reinterpret_cast<const float4*>(bp + r0) : zero4;
+        b1[j] = ok && r1 < lo.rank ? *reinterpret_cast<const float4*>(bp + r1) : zero4;
     }
     const float sc = F32 ? lo.scale : (float)(__bf16)lo.scale;
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int i = 0; i < kMT; ++i) {
-        const float* tp = ts + (16 * i + col) * lo.rank + r0;
-        const float4 t0 = r0 < lo.rank ? *reinterpret_cast<const float4*>(tp) : zero4;
-        const float4 t1 = r0 + 4 < lo.rank ? *reinterpret_cast<const float4*>(tp + 4) : zero4;
-        bf16x8 th, tl;
-        split_bf16x8(t0, t1, th, tl);
+        const float* tp = ts + (16 * i + col) * lo.rank;
+        const float4 t0 = r0 < lo.rank ? *reinterpret_cast<const float4*>(tp + r0) : zero4;
+        const float4 t1 = r1 < lo.rank ? *reinterpret_cast<const float4*>(tp + r1) : zero4;
 #pragma unroll
         for (int j = 0; j < kNT; ++j) {
-            f32x4 d = mfma16x16x32(th, bh[j], zero);
-            d = mfma16x16x32(th, bl[j], d);
-            d = mfma16x16x32(tl, bh[j], d);
+            f32x4 d = mfma16x16x4(t0.x, b0[j].x, zero);
+            d = mfma16x16x4(t0.y, b0[j].y, d);
+            d = mfma16x16x4(t0.z, b0[j].z, d);
+            d = mfma16x16x4(t0.w, b0[j].w, d);
+            if (lo.rank > 16) {
+                d = mfma16x16x4(t1.x, b1[j].x, d);
+                d = mfma16x16x4(t1.y, b1[j].y, d);
+                d = mfma16x16x4(t1.z, b1[j].z, d);
+                d = mfma16x16x4(t1.w, b1[j].w, d);
+            }
             const int n = (rb0 + j) * 16 + col;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
