@@ -1,5 +1,5 @@
 // Decode-shape affine-Q4 matmul on gfx950: y[M,N] = x[M,K] . W^T for M <= 16 (and
-// beyond, for weights small enough that slabs beat the GEMM's fixed costs), in
+// beyond, up to 31 rows and for small weights, see use_decode in q4_kernels.h), in
 // 16-row slabs (one launch; slab = blockIdx.y).
 //
 // Bandwidth-bound: every weight byte is read once from HBM with 16-byte coalesced

@@ -206,38 +206,63 @@ hipError_t launch_lora(const uint16_t* x, const float* a, const uint16_t* a_hi, 
 hipError_t launch_lora_down(const uint16_t* x, const uint16_t* a_hi, const uint16_t* a_lo, float* part, int m,
                             int k, int rank, hipStream_t stream);
 
-// Forward path choice (automatic mode): the decode kernels up to 16 rows (one slab),
-// and beyond that while 16-row slabs x N x K stays at most kDecodeMaxSlabWork (K' = 2K
-// for two-plane 8-bit handles).  The decode kernels' cost grows by one pass over the
-// weights per 16-row slab (~0.24 us per million weights); the GEMM's starts at ~10 us
-// (launch, tile prologue and epilogue, split-K reduction) and grows slowly at these
-// sizes.  Measured as whole forwards (graph replays over rotated weight copies, each
-// path pinned) on eight shapes at 8-400 rows, decode / GEMM in us:
-//   up to the bound: o 3840x4096 at 17 rows 9.1 / 10.9, at 32 11.5 / 11.4; k 2048x3840 at
-//     64 11.0 / 11.8; the full-attention k 512x3840 at 256 10.8 / 11.8;
-//   past it: q 4096x3840 at 40 13.9 / 12.8; k at 96 14.9 / 12.9; qkv 8192x3840 at 17
-//     15.4 / 10.3; the gate|up pair at 17 38.5 / 23.9; down at 17 29.9 / 17.6.
-// (Up to 16 rows decode is ahead or within 15%: qkv at 16 11.4 / 10.3, the pair 21.7 / 24.1.)
-constexpr int kGemmMinRows = 17;
+// Forward path choice (automatic mode).
+//
+// Up to 31 rows, and beyond that while 16-row slabs x N x K' stays at most
+// kScratchFreeSlabWork (K' = 2K for two-plane 8-bit handles), a plain forward takes no
+// scratch: such calls may be captured on a stream the library has not seen, graphs of
+// them captured on one stream may be replayed side by side, and they may overlap through
+// the allocation-free entry point.  They run on the decode kernels, or on a GEMM plan that
+// needs no scratch (K unsplit) where that is the faster of the two.
+//
+// The decode kernels cost one pass over the weights per slab; a GEMM with K unsplit costs
+// some 2 us per 256 columns of K on up to 256 output tiles of 256 columns.  So N times the
+// slabs decides.  Measured as whole forwards (graph replays over rotated weight copies,
+// each path pinned), decode / unsplit GEMM in us:
+//   4 bits, past 16 rows: below the line gate 15360x3840 at 17 rows 25.6 / 31.1, qkv
+//     8192x3840 16.9 / 30.6, q 4096x3840 at 48 15.9 / 26.1; past it 24576x3840 at 17
+//     33.9 / 31.9, the gate|up pair 43.2 / 33.4, 32768x2048 29.3 / 19.7, 65536x512 20.1 / 9.2,
+//     16384x1024 at 33 14.6 / 10.3.
+//   8 bits from 9 rows: 65536x3840 at 9 114 / 78; 65536x1024 even to 12 rows (22.9 / 23.7),
+//     at 16 30.5 / 23.4; the pair at 9 57 / 61.
+//   8 bits from 12 rows: below the line 24576x3840 at 16 57.1 / 59.4, down 3840x15360 38.8 /
+//     211, qkv at 31 37.9 / 56.6; past it the pair at 12 64.7 / 60.9, at 31 135 / 61.5,
+//     gate at 17 58.5 / 57.8, at 31 71.7 / 58.0.
+// (A split of K would be faster on most of them: the pair at 17 rows 25.1 us, qkv 11.8, the
+// 8-bit pair at 16 40.7.  Its partial sums are the scratch.)
+//
+// Past the scratch-free calls the GEMM's fixed cost is ~10 us: decode / GEMM o 3840x4096 at
+// 48 rows 15.3 / 13.3, at 64 19.4 / 14.4; qkv at 32 19.7 / 11.1, at 48 28.1 / 12.8.
+constexpr int kScratchFreeRows = 31;
+constexpr double kScratchFreeSlabWork = 5.5e7;
+constexpr long kScratchFreeMaxRows = 1024;
+// While the slabs' work stays at most this, the decode kernels are taken without asking for
+// the GEMM (o at 32 rows 11.5 / 11.4 with a split; k 2048x3840 at 64 11.0 / 11.8).
 constexpr double kDecodeMaxSlabWork = 3.5e7;
-// From 9 rows a two-plane 8-bit handle's x' no longer fits the decode kernels' LDS beside
-// its steps, and with enough weights the GEMM is ahead there, too (decode / GEMM, us, at
-// 9, 12 and 16 rows): gate 27.8 / 23.6, 32.2 / 23.8, 38.0 / 23.9; the pair 52.9 / 38.8,
-// 61.7 / 39.0, 73.4 / 40.1; down 27.4 / 26.1, 32.4 / 26.0, 38.3 / 26.2; from 12 rows with
-// fewer: qkv 8192x3840 15.3 / 14.9, 17.6 / 15.0, 20.5 / 15.0; the full-attention o
-// 3840x8192 14.9 / 17.2, 17.2 / 17.2, 19.6 / 17.3; not o 3840x4096 (11.4 / 14.0 at 16).
+// Slabs x N from which the unsplit GEMM is taken: 4 bits past 16 rows; 8 bits from 9 and
+// from 12 rows.
+constexpr double kUnsplitCols = 4.5e4;
 constexpr int kTwoPlaneRows[2] = {9, 12};
-constexpr double kTwoPlaneWork[2] = {1.0e8, 6.0e7};  // N x K' from that many rows on
-// Beyond 64 slabs the GEMM takes any shape.
-constexpr long kDecodeMaxRows = 1024;
+constexpr double kTwoPlaneUnsplitCols[2] = {6.0e4, 3.0e4};
+
+inline double slab_work(long rows, const Layout& l) {
+    return (double)((rows + 15) / 16) * (double)l.n * (double)l.k;
+}
+inline bool scratch_free(long rows, const Layout& l) {
+    return rows <= kScratchFreeRows || (rows <= kScratchFreeMaxRows && slab_work(rows, l) <= kScratchFreeSlabWork);
+}
 inline bool use_decode(long rows, const Layout& l, int gemm_min_rows) {
     if (gemm_min_rows > 0) return rows < gemm_min_rows;
-    if (rows < kGemmMinRows) {
-        if (l.kx == l.k || rows < kTwoPlaneRows[0]) return true;
-        return (double)l.n * (double)l.k < kTwoPlaneWork[rows < kTwoPlaneRows[1] ? 0 : 1];
-    }
-    return rows <= kDecodeMaxRows &&
-           (double)((rows + 15) / 16) * (double)l.n * (double)l.k <= kDecodeMaxSlabWork;
+    if (!scratch_free(rows, l)) return false;
+    const bool two_plane = l.kx != l.k;
+    if (rows < (two_plane ? kTwoPlaneRows[0] : 17) || slab_work(rows, l) <= kDecodeMaxSlabWork) return true;
+    const double cols = (double)((rows + 15) / 16) * (double)l.n;
+    return cols < (two_plane ? kTwoPlaneUnsplitCols[rows < kTwoPlaneRows[1] ? 0 : 1] : kUnsplitCols);
+}
+// Scratch the GEMM of such a call may plan with: none for the scratch-free calls (a pinned
+// path plans freely).
+inline size_t gemm_room(long rows, const Layout& l, int gemm_min_rows) {
+    return gemm_min_rows == 0 && scratch_free(rows, l) ? 0 : ~(size_t)0;
 }
 
 }  // namespace q4

@@ -523,7 +523,8 @@ Gemma4Status dispatch_forward(const Gemma4QLinear* linear, const uint16_t* x_dev
     const int mode = geglu ? (f32 ? q4::kOutGegluF32 : q4::kOutGegluBf16) : (f32 ? q4::kOutF32 : q4::kOutBf16);
     const int n_out = linear->pair_rows;
     hipError_t e;
-    if (q4::use_decode(rows, linear->layout, (int)g_gemm_min_rows.load(std::memory_order_relaxed))) {
+    const int min_rows = (int)g_gemm_min_rows.load(std::memory_order_relaxed);
+    if (q4::use_decode(rows, linear->layout, min_rows)) {
         const q4::OutParams op{y_dev, nullptr, mode, n_out, 0, 0.0f};
         e = q4::launch_decode(linear->tiles, linear->sb, x_dev, op, (int)rows, linear->layout, sc.stream);
         if (e != hipSuccess) return hip_fail((name + ": decode launch").c_str(), e);
@@ -534,9 +535,10 @@ Gemma4Status dispatch_forward(const Gemma4QLinear* linear, const uint16_t* x_dev
     // only tiles and splits that fit that room; an unsplit plan of 64- or 128-row tiles
     // needs none)
     const q4::Layout gl = gemm_layout(linear);
-    size_t ws_bytes = q4::gemm_workspace_bytes((int)rows, gl);
+    const size_t room = q4::gemm_room(rows, gl, min_rows);
+    size_t ws_bytes = q4::plan_gemm((int)rows, gl, room).total();
     if (sc.fixed) {
-        ws_bytes = sc.room();
+        ws_bytes = sc.room() < room ? sc.room() : room;
         // holds by construction (the plan takes only what fits the room); kept so that
         // a plan change can never overrun the array
         const q4::GemmPlan plan = q4::plan_gemm((int)rows, gl, ws_bytes);
@@ -844,9 +846,10 @@ Gemma4Status gemma4_qlinear_scratch_bytes(const Gemma4QLinear* linear, uint32_t 
         if (!valid_handle(linear))
             return fail(GEMMA4_ERR_INVALID_ARGUMENT, "gemma4_qlinear_scratch_bytes received an invalid handle");
         *out = 0;
-        if (rows == 0 || q4::use_decode(rows, linear->layout, (int)g_gemm_min_rows.load(std::memory_order_relaxed)))
-            return ok();
-        *out = q4::gemm_workspace_bytes((int)rows, gemm_layout(linear));
+        const int min_rows = (int)g_gemm_min_rows.load(std::memory_order_relaxed);
+        if (rows == 0 || q4::use_decode(rows, linear->layout, min_rows)) return ok();
+        const q4::Layout gl = gemm_layout(linear);
+        *out = q4::plan_gemm((int)rows, gl, q4::gemm_room(rows, gl, min_rows)).total();
         return ok();
     } catch (...) {
         return fail_nothrow(GEMMA4_ERR_RUNTIME, "gemma4_qlinear_scratch_bytes: unexpected native exception");

@@ -120,13 +120,15 @@ Gemma4Status gemma4_qmm_get_last_error(char* buffer, size_t buffer_len);
 
 /* Path choice of the forward calls in this process.  No counterpart in the
  * reference (MLX picks its own kernels); for tests and benchmarks that pin a path.
- *   0 (the default): automatic.  The decode kernels (16-row slabs, one pass over
- *     the weights per slab) up to 16 rows, and beyond that while
- *     ceil(rows / 16) * N * K <= 3.5e7 (K' = 2K for 8-bit handles), the GEMM
- *     otherwise: for the Gemma 4 shapes the decode kernels are ahead of the GEMM's
- *     fixed costs up to 32 rows for 4096x3840, 64 for 2048x3840, 272 for 512x3840,
- *     and up to 16 rows for 8192x3840 and the MLP projections.  8-bit handles go
- *     to the GEMM from 9 rows with N * K' >= 1e8 and from 12 with N * K' >= 6e7.
+ *   0 (the default): automatic.  Calls of up to 31 rows, and of up to 1024 while
+ *     ceil(rows / 16) * N * K' <= 5.5e7 (K' = 2K for 8-bit handles), take no scratch:
+ *     they run on the decode kernels (16-row slabs, one pass over the weights per
+ *     slab) or, on wide outputs, on the GEMM with K unsplit (from 17 rows with
+ *     ceil(rows / 16) * N >= 4.5e4; 8-bit handles from 9 rows with 6e4 and from 12
+ *     with 3e4; never while the slabs' work is at most 3.5e7).  For the Gemma 4
+ *     shapes: the decode kernels up to 48 rows for 4096x3840, 96 for 2048x3840, 432
+ *     for 512x3840 and 31 for 8192x3840, gate and down; up to 16 for the gate|up
+ *     pair.  The GEMM with any plan otherwise.
  *   r > 0: the GEMM from r rows on, the decode kernels below.
  * Both paths meet the same accuracy contract; they sum in different orders, so the
  * last bits of some outputs differ between them.  Returns the previous setting.

@@ -1,6 +1,6 @@
 """8-bit handles at the row counts where their path changes: 2 to 5 rows (the int8 kernels
 up to 2, the bf16 ones from 3) and 8 to 17 rows around the
-GEMM's first (9 rows from N x 2K = 1e8, 12 from 6e7).  Every automatic result against the oracle and
+first row counts at which wide outputs go to the GEMM (9 and 12).  Every automatic result against the oracle and
 against both pinned paths: fp32 outputs within GEMM_REL of the RMS (the kernels' sums are
 exact products in fp32, in different orders)."""
 

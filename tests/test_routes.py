@@ -1,0 +1,50 @@
+"""Path choice of the forward calls (CPU: the library's own rule and plan, no launch).
+
+A plain forward of up to 31 rows, and of up to 1024 while ceil(rows / 16) * N * K' <= 5.5e7
+(K' = 2K for 8-bit handles), takes no scratch: such calls are captured on cold streams, their
+graphs replayed side by side, and they overlap through the allocation-free entry point."""
+
+import itertools
+
+import pytest
+
+from plan_host import route
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+def test_scratch_free_calls_take_no_scratch(bits):
+    rows = (1, 2, 3, 8, 9, 11, 12, 15, 16, 17, 24, 31, 32, 33, 48, 49, 64, 96, 112, 113, 256, 272, 432, 1000, 1024, 1025)
+    free = paths = 0
+    for n, k, m in itertools.product((16, 100, 512, 1000, 2048, 3840, 4096, 8192, 15360, 24576, 65536, 262144),
+                                     (64, 576, 1024, 3840, 4096, 8192, 15360), rows):
+        work = -(-m // 16) * n * k * (bits // 4)
+        if m > 31 and (m > 1024 or work > 5.5e7):
+            continue
+        free += 1
+        for pair in (False, True) if n <= 65536 else (False,):
+            if pair and m > 31 and 2 * work > 5.5e7:
+                continue
+            r = route(n, k, m, bits=bits, pair=pair)
+            paths += r["decode"]
+            assert r["decode"] or (r["scratch"] == 0 and r["splits"] == 1), (n, k, m, bits, pair, r)
+    assert free > 500 and paths > 500
+
+
+@pytest.mark.parametrize("n,k,bits,pair,rows,decode", [
+    (8192, 3840, 4, False, 17, True), (8192, 3840, 4, False, 31, True), (8192, 3840, 4, False, 32, False),
+    (15360, 3840, 4, False, 17, True), (15360, 3840, 4, True, 16, True), (15360, 3840, 4, True, 17, False),
+    (4096, 3840, 4, False, 48, True), (4096, 3840, 4, False, 49, False), (2048, 3840, 4, False, 96, True),
+    (2048, 3840, 4, False, 97, False), (512, 3840, 4, False, 432, True), (16384, 1024, 4, False, 33, False), (65536, 512, 4, False, 17, False),
+    (15360, 3840, 8, True, 11, True), (15360, 3840, 8, True, 12, False), (15360, 3840, 8, False, 16, True),
+    (15360, 3840, 8, False, 17, False), (65536, 3840, 8, False, 8, True), (65536, 3840, 8, False, 9, False),
+    (3840, 15360, 8, False, 31, True), (3840, 15360, 8, False, 32, False)])
+def test_route_edges(n, k, bits, pair, rows, decode):
+    """Both sides of each line of the rule."""
+    assert bool(route(n, k, rows, bits=bits, pair=pair)["decode"]) == decode
+
+
+def test_pinned_path_plans_freely():
+    """gemm_min_rows pins the GEMM with its whole plan, scratch included."""
+    r = route(8192, 3840, 17, min_rows=1)
+    assert not r["decode"] and r["splits"] > 1 and r["scratch"] > 0
+    assert route(15360, 3840, 700, min_rows=1 << 20)["decode"]
