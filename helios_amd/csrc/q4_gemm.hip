@@ -1046,21 +1046,14 @@ GemmPlan plan_gemm(int m, const Layout& l, size_t max_workspace) {
     return p;
 }
 
-size_t gemm_workspace_bytes(int m, const Layout& l) { return plan_gemm(m, l).total(); }
-
 hipError_t launch_gelu_table(uint16_t* table, hipStream_t stream) {
     hipLaunchKernelGGL(gelu_table_kernel, dim3((kGeluTable + 255) / 256), dim3(256), 0, stream, table);
     return hipGetLastError();
 }
 
-bool gemm_lora_epilogue(int m, const Layout& l, int rank, size_t workspace_bytes) {
-    return rank >= 4 && rank <= 32 && rank % 4 == 0 && plan_gemm(m, l, workspace_bytes).splits == 1;
-}
-
 hipError_t launch_gemm(const uint4* tiles, const uint2* sb, const uint16_t* x, void* y, int m, int out_mode,
-                       int n_out, const Layout& l, void* workspace, size_t workspace_bytes,
+                       int n_out, const Layout& l, const GemmPlan& plan, void* workspace, size_t workspace_bytes,
                        const uint16_t* gelu_table, hipStream_t stream, const LoraEpilogue* lora) {
-    const GemmPlan plan = plan_gemm(m, l, workspace_bytes);
     if (plan.total() > workspace_bytes) return hipErrorInvalidValue;
     const LoraEpilogue lo = lora != nullptr ? *lora : LoraEpilogue{nullptr, nullptr, 0, 0, 0.0f};
     if (lora != nullptr && (plan.splits != 1 || out_mode > kOutF32 || lo.rank % 4 != 0 || lo.rank < 4 ||
@@ -1114,7 +1107,7 @@ hipError_t launch_gemm(const uint4* tiles, const uint2* sb, const uint16_t* x, v
             const hipError_t ek = launch_kpair(tiles, sb, x, YPTR, m, MODE, n_out, l, plan, STRIDE, gelu_table,  \
                                                lo, stream);                                                      \
             if (ek != hipSuccess) return ek;                                                                     \
-        } else if (plan.bm == 64)                                                                                       \
+        } else if (plan.bm == 64)                                                                                \
             hipLaunchKernelGGL((gemm_kernel<MODE, 64, 256>), grid, block, 0, stream, Q4_GEMM_ARGS(YPTR, STRIDE));  \
         else if (plan.bm == 256 && plan.f16)                                                                     \
             hipLaunchKernelGGL((gemm_kernel<MODE, 256, 256, 1>), grid, block, 0, stream,                         \

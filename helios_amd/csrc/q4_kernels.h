@@ -137,10 +137,9 @@ void set_f16_form(Layout& l, const int range[3]);
 // for the 256-row tile and the pre-pass forms (fp16 on 256-row tiles, one-pass 8-bit
 // on 128- and 256-row tiles), the group sums of x (and in the pre-pass forms x as
 // fp16 and each row's power of two) and, when K is split over workgroups, the fp32
-// partial sums (device memory, 256-byte aligned); an unsplit bf16-form plan of 64- or
+// partial sums (device memory, 256-byte aligned); an unsplit bf16-form plan of 32- to
 // 128-row tiles needs none.  The plan is the cheapest whose workspace fits in
-// `workspace_bytes`; gemm_workspace_bytes(m, l) is what the unconstrained plan
-// needs, and with that much the launch runs the unconstrained plan.
+// `max_workspace`; a call makes it once (0.8 to 1.5 us of host time) and hands it on.
 struct GemmPlan {
     int bm = 256;            // output tile rows
     int bn = 256;            // output tile columns
@@ -158,14 +157,13 @@ struct GemmPlan {
 constexpr int kMaxSplits = 16;
 constexpr size_t kMaxPartialBytes = (size_t)1 << 30;
 GemmPlan plan_gemm(int m, const Layout& l, size_t max_workspace = ~(size_t)0);
-size_t gemm_workspace_bytes(int m, const Layout& l);
 
 // Compute units of the current device (cached per device).
 int device_cus();
 // gelu_table: kGeluTable bf16 values (q4_common.h) from launch_gelu_table, staged in
 // LDS by the bf16 GeGLU epilogue (out_mode 2); may be null for the other modes.
 hipError_t launch_gemm(const uint4* tiles, const uint2* sb, const uint16_t* x, void* y, int m, int out_mode,
-                       int n_out, const Layout& l, void* workspace, size_t workspace_bytes,
+                       int n_out, const Layout& l, const GemmPlan& plan, void* workspace, size_t workspace_bytes,
                        const uint16_t* gelu_table, hipStream_t stream, const LoraEpilogue* lora = nullptr);
 // One launch of a kpair plan (q4_gemm_kpair.hip): y in out_mode (a mode of the GEMM), or
 // the partial planes of a split; lora only in the LoRA modes.
@@ -180,9 +178,10 @@ inline bool kpair_fits(int m, const Layout& l) {
     return ((size_t)m + kKpairMaxRows) * l.kx * 2 < wrap && l.rec_bytes() + (size_t)16 * l.gp * kRecBytes < wrap &&
            l.rec_bytes() <= kMaxRecBytes && (size_t)kKpairMaxRows * l.n * 4 < kMaxRecBytes;
 }
-// Whether launch_gemm can add a LoRA delta of this rank in its epilogue for m rows
-// within `workspace_bytes` (an unsplit plan; rank a multiple of 4 up to 32).
-bool gemm_lora_epilogue(int m, const Layout& l, int rank, size_t workspace_bytes);
+// Whether the plan's launch can add a LoRA delta of this rank in its epilogue.
+inline bool gemm_lora_epilogue(const GemmPlan& plan, int rank) {
+    return plan.splits == 1 && rank >= 4 && rank <= 32 && rank % 4 == 0;
+}
 
 // Fills table[kGeluTable] with gelu of the bf16 patterns that need a table, in the
 // bf16 op sequence.

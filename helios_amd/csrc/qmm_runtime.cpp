@@ -530,31 +530,22 @@ Gemma4Status dispatch_forward(const Gemma4QLinear* linear, const uint16_t* x_dev
         if (e != hipSuccess) return hip_fail((name + ": decode launch").c_str(), e);
         return GEMMA4_OK;
     }
-    // group sums of x (256-row tiles) and split-K partial sums: the unconstrained plan's
-    // workspace from the pool, or what the static scratch has left (the plan then takes
-    // only tiles and splits that fit that room; an unsplit plan of 64- or 128-row tiles
-    // needs none)
+    // group sums of x (256-row tiles), the pre-pass forms' x and split-K partial sums: the
+    // unconstrained plan's from the stream's memory, or what the static scratch has left
+    // (the plan then takes only tiles and splits that fit that room, so it cannot overrun
+    // the array; an unsplit bf16-form plan of 32- to 128-row tiles needs none), and none
+    // for the scratch-free calls
     const q4::Layout gl = gemm_layout(linear);
-    const size_t room = q4::gemm_room(rows, gl, min_rows);
-    size_t ws_bytes = q4::plan_gemm((int)rows, gl, room).total();
-    if (sc.fixed) {
-        ws_bytes = sc.room() < room ? sc.room() : room;
-        // holds by construction (the plan takes only what fits the room); kept so that
-        // a plan change can never overrun the array
-        const q4::GemmPlan plan = q4::plan_gemm((int)rows, gl, ws_bytes);
-        if (plan.total() > ws_bytes)
-            return fail(GEMMA4_ERR_UNSUPPORTED_CONFIG, name + ": the GEMM's scratch needs more than the " +
-                                                           std::to_string(kStaticScratchBytes) +
-                                                           "-byte static scratch has left");
-    }
+    const size_t most = q4::gemm_room(rows, gl, min_rows);
+    const q4::GemmPlan plan = q4::plan_gemm((int)rows, gl, sc.room() < most ? sc.room() : most);
+    const size_t ws_bytes = plan.total();
     void* ws = nullptr;
-    e = sc.take(sc.fixed ? 0 : ws_bytes, &ws);
-    if (sc.fixed) ws = sc.base + sc.used;
+    e = sc.take(ws_bytes, &ws);
     if (e != hipSuccess)
         return fail(GEMMA4_ERR_MEMORY_GUARD, name + ": workspace allocation failed: " + hipGetErrorString(e));
     q4::LoraEpilogue lo{};
     const bool with_lora = lora != nullptr && !geglu && !sc.fixed &&
-                           q4::gemm_lora_epilogue((int)rows, gl, (int)lora->rank, ws_bytes);
+                           q4::gemm_lora_epilogue(plan, (int)lora->rank);
     if (with_lora) {
         const int slices = q4::lora_slices((int)linear->desc.in_features, (int)rows);
         void* part = nullptr;
@@ -566,7 +557,7 @@ Gemma4Status dispatch_forward(const Gemma4QLinear* linear, const uint16_t* x_dev
         if (e != hipSuccess) return hip_fail((name + ": lora_down launch").c_str(), e);
         lo = q4::LoraEpilogue{static_cast<const float*>(part), lora->b, (int)lora->rank, slices, lora->scale};
     }
-    e = q4::launch_gemm(linear->tiles, linear->sb, x_dev, y_dev, (int)rows, mode, n_out, gl, ws, ws_bytes,
+    e = q4::launch_gemm(linear->tiles, linear->sb, x_dev, y_dev, (int)rows, mode, n_out, gl, plan, ws, ws_bytes,
                         linear->gelu_table, sc.stream, with_lora ? &lo : nullptr);
     if (e != hipSuccess) return hip_fail((name + ": gemm launch").c_str(), e);
     if (lora_done != nullptr) *lora_done = with_lora;
