@@ -8,8 +8,8 @@
 //   acc += 16*s * P_g on the fp32 accumulators (one VALU FMA per output per group);
 // * the bias term: one extra MFMA per tile per 8 groups on an augmented K of 32,
 //   A = [Xh, Xl, -16Xh, -16Xl] per group (X_g = Xh + Xl split into two bf16),
-//   B = [b, b, s, s] taken straight from the scale/bias words.  In the 64- and
-//   128-row tiles X_g comes from the x tile in LDS: two MFMAs of an all-ones A
+//   B = [b, b, s, s] taken straight from the scale/bias words.  In the 128-row
+//   tile X_g comes from the x tile in LDS: two MFMAs of an all-ones A
 //   against a row tile's x fragments (as B) sum the group's 64 values of its 16 rows,
 //   each wave for its own row tiles.  The 256-row tile takes it from xaug_kernel, a
 //   pre-pass: there every wave reads the 256 rows' fragments from LDS already (about
@@ -34,12 +34,11 @@
 //
 // Tiling: a 512-thread workgroup computes a 256 (M) x 256 (N) tile as eight waves
 // side by side along N, each all 256 rows x 32 columns (two waves per SIMD, so one's
-// MFMA and LDS latencies are covered by the other's work); or 128 x 256, or 64 x 256
-// (eight waves of 128 or 64 x 32).  A wave expands only its own two row blocks'
+// MFMA and LDS latencies are covered by the other's work); or 128 x 256
+// (eight waves of 128 x 32).  A wave expands only its own two row blocks'
 // nibbles and reads every x row of the tile from LDS: expansion is VALU work and was
 // the wider cost (measured against 2 x 4 waves of BM/2 x 64, with bit-identical
-// results: the 64-row tile 8-13% faster, the 128-row tile 3-9%, the 256-row tile
-// 0-6%).  The kernel is written
+// results: the 128-row tile 3-9% faster, the 256-row tile 0-6%).  The kernel is written
 // for tiles of BN = 128 too (four waves, 78 KiB of LDS: two workgroups per CU); a
 // forced-plan sweep over the benchmark's shapes measured it within 6% of the two
 // tiles above where it helped at all, so the plan does not use it.  Everything streams
@@ -280,16 +279,14 @@ __global__ __launch_bounds__(BN * 2) void gemm_kernel(const uint4* __restrict__ 
                                                    const uint16_t* __restrict__ gelu_table, LoraEpilogue lora,
                                                    const int* __restrict__ rowexp, float s_pow, int lo_pairs) {
     // BN / 32 waves of BM x 32: BM = 256; BM = 128 (more workgroups for small M
-    // without splitting K); BM = 64 (fewest K splits for narrow outputs).  FORM 1 and 2:
-    // x is x16, rowexp from the pre-pass; FORM 1: s_pow = 2^p of the handle; FORM 2:
+    // without splitting K).  FORM 1 and 2: x is x16, rowexp from the pre-pass; FORM 1: s_pow = 2^p of the handle; FORM 2:
     // groups and pairs count the original K (the high plane), the low plane's pair p
     // is record lo_pairs + p.
-    static_assert(BM == 256 || BM == 128 || BM == 64, "tile rows");
+    static_assert(BM == 256 || BM == 128, "tile rows");
     static_assert(BN == 256 || BN == 128, "tile columns");
     constexpr bool F16 = FORM == 1;
     constexpr bool kQ8 = FORM == 2;
     static_assert(!F16 || BM == 256, "the fp16 form takes its group sums from the pre-pass");
-    static_assert(!kQ8 || BM >= 128, "one-pass 8-bit: 128- and 256-row tiles");
     // x ring slots: three (a group's x loaded two steps ahead), or two (one step ahead)
     // where two planes' words per weight slot leave no room for a third 32 KiB slot
     // (one-pass 8-bit at 256 rows: 156 KiB against 188)
@@ -303,18 +300,17 @@ __global__ __launch_bounds__(BN * 2) void gemm_kernel(const uint4* __restrict__ 
     constexpr int kXaA = BM / 16 * 64;            // uint4: the bias A operands of the tile's rows
     constexpr int kMT = BM / 16;                  // 16x16 tiles per wave along M
     constexpr int kXParts = BM * 8 / (64 * kWaves);  // 16-byte x loads per wave per group
-    // X_g summed in the kernel (64 and 128 rows), or read from xaug (256 rows, and every
+    // X_g summed in the kernel (128 rows), or read from xaug (256 rows, and every
     // tile of the pre-pass forms)
     constexpr bool kXIn = BM < 256 && FORM == 0;
-    // in the kernel: row tiles whose X_g a wave sums, tiles wave + 8t (BM = 64: waves
-    // 0-3 one each, the rest none)
+    // in the kernel: row tiles whose X_g a wave sums, tiles wave + 8t
     constexpr int kXTiles = kXIn ? (kMT + kWaves - 1) / kWaves : 0;
     // from xaug: 16-byte loads of bias A operands per wave per octet
     constexpr int kXaParts = BM / 16 / kWaves;
     constexpr int kSWaves = kRB / 8;              // waves that load a pair's scale words (1 KiB each)
-    constexpr int kTW = kMT * kNT >= 12 ? 9 : 5;  // product-stream tile after which a pair's weights are issued
+    constexpr int kTW = 9;                        // product-stream tile after which a pair's weights are issued
     static_assert(kRB == 2 * kWaves, "two row blocks of tiled words per wave per pair");
-    static_assert(kXParts >= 1 && (kXIn ? kMT <= kXTiles * kWaves : kXaParts * kWaves == kMT),
+    static_assert(kXParts >= 1 && (kXIn ? kMT == kXTiles * kWaves : kXaParts * kWaves == kMT),
                   "every wave loads x; every row tile's X_g is summed or loaded");
     __shared__ uint4 g_xs0[kXChunks];             // x group tiles (BM rows x 64: 16 or 32 KiB)
     __shared__ uint4 g_xs1[kXChunks];
@@ -462,7 +458,7 @@ __global__ __launch_bounds__(BN * 2) void gemm_kernel(const uint4* __restrict__ 
         // (B[k][n] = x[16i + n][k]) against ones, so every output of column n is the sum
         // of row n's 64 values.  Read again here rather than taken from the product
         // stream, which would need a branch per row tile.
-        if (kXIn && (kMT % kWaves == 0 || wave < kMT)) {
+        if (kXIn) {
 #pragma unroll
             for (int t = 0; t < kXTiles; ++t) {
                 const bf16x8 b0 = a_frag(wave + kWaves * t, 0), b1 = a_frag(wave + kWaves * t, 1);
@@ -633,7 +629,7 @@ __global__ __launch_bounds__(BN * 2) void gemm_kernel(const uint4* __restrict__ 
         compute(xs, wp, g & 1, [&](int t) {
             if ((t & 1) && (t >> 1) < kXParts) dma_x(g + kXSlots - 1, t >> 1, xs2);
             // the pair's two weight loads after tiles kTW and kTW + 2 (inside the stream
-            // of kMT x kNT tiles: 8 of them for 64-row tiles)
+            // of kMT x kNT tiles)
             if (pair && (t == kTW || t == kTW + 2)) dma_w((g + 2) >> 1, (t - kTW) >> 1, wp2);
         });
         // lane (col, kq) keeps X_g of groups 2kq and 2kq + 1 of the octet
@@ -923,14 +919,13 @@ struct TileShape {
     int bm, bn;
     bool kpair;  // q4_gemm_kpair.hip
 };
-// The bf16 form on 64-row tiles is behind the kpair tiles in every case measured (at 64
-// rows qkv 16.7 us against 12.8, the pair 33.2 against 31.5; at 1100 rows 107 against 85
-// and 331 against 282) and is offered only to handles those cannot address; the 128-row
-// tile is ahead of them where it leaves no round short (the pair at 256 rows 74.5 against
-// 77.6).
-constexpr TileShape kTileShapes[] = {{256, 256, false}, {128, 256, false}, {64, 256, false}, {32, 256, true},
-                                     {48, 256, true},   {64, 256, true},   {80, 256, true},  {96, 256, true},
-                                     {112, 256, true}};
+// The 128-row tile is ahead of the kpair tiles where it leaves no round short (the pair at
+// 256 rows 74.5 us against 77.6) and takes every shape those cannot address (kpair_fits:
+// N above some 4.7 million).  A 64-row tile of its kind was behind them in every case
+// measured (at 64 rows qkv 16.7 us against 12.8, the pair 33.2 against 31.5; at 1100 rows
+// 107 against 85 and 331 against 282) and is gone.
+constexpr TileShape kTileShapes[] = {{256, 256, false}, {128, 256, false}, {32, 256, true}, {48, 256, true},
+                                     {64, 256, true},   {80, 256, true},   {96, 256, true}, {112, 256, true}};
 constexpr double kFill = 0.426;
 constexpr double kSplitUs = 3.8, kPerSplitUs = 0.38;  // a split's reduction launch
 constexpr double kPartialBytesPerUs = 17.0e6;         // partial sums written and read back, mostly in the caches
@@ -944,7 +939,7 @@ double body_us(const TileShape& ts, double step_scale, int groups) {
         const double mt = ts.bm / 16;
         return groups / 4.0 * (0.693 + 0.261 * mt) + 0.737 * mt;
     }
-    const double step = ts.bm == 256 ? 1.202 : ts.bm == 128 ? 0.766 : 0.46;
+    const double step = ts.bm == 256 ? 1.202 : 0.766;
     return groups * step * step_scale + 1.464 * (1.0 + ts.bm / 64.0);
 }
 // the fp16 form: its group step against the bf16 form's (gate 15360x3840 at 2048 rows,
@@ -995,12 +990,12 @@ GemmPlan plan_gemm(int m, const Layout& l, size_t max_workspace) {
     double best = -1.0;
     for (const TileShape& ts : kTileShapes) {
         const int bm = ts.bm, bn = ts.bn;
-        if (ts.kpair ? !kp : (bm == 64 && kp)) continue;
+        if (ts.kpair && !kp) continue;
         const long tiles = (long)((m + bm - 1) / bm) * ((l.n + bn - 1) / bn);
         // form 0: the bf16 form; 1: the fp16 form (256-row tiles of handles whose scales
         // allow it); 2: one-pass 8-bit (128- and 256-row tiles)
         for (int form = 2; form >= 0; --form) {
-            if ((form == 1 && !(bm == 256 && l.f16 && l.prepass_forms)) || (form == 2 && !(bm >= 128 && q8_ok)) ||
+            if ((form == 1 && !(bm == 256 && l.f16 && l.prepass_forms)) || (form == 2 && !q8_ok) ||
                 (form != 0 && ts.kpair))
                 continue;
             const bool pre = form != 0;
@@ -1107,9 +1102,7 @@ hipError_t launch_gemm(const uint4* tiles, const uint2* sb, const uint16_t* x, v
             const hipError_t ek = launch_kpair(tiles, sb, x, YPTR, m, MODE, n_out, l, plan, STRIDE, gelu_table,  \
                                                lo, stream);                                                      \
             if (ek != hipSuccess) return ek;                                                                     \
-        } else if (plan.bm == 64)                                                                                \
-            hipLaunchKernelGGL((gemm_kernel<MODE, 64, 256>), grid, block, 0, stream, Q4_GEMM_ARGS(YPTR, STRIDE));  \
-        else if (plan.bm == 256 && plan.f16)                                                                     \
+        } else if (plan.bm == 256 && plan.f16)                                                                   \
             hipLaunchKernelGGL((gemm_kernel<MODE, 256, 256, 1>), grid, block, 0, stream,                         \
                                Q4_GEMM_ARGS(YPTR, STRIDE));                                                      \
         else if (plan.bm == 128 && plan.q8)                                                                      \

@@ -219,7 +219,7 @@ Gemma4Status gemma4_qlinear_scratch_bytes(const Gemma4QLinear* linear, uint32_t 
  * sums, only as far as the array has room (a cheaper tile, another form or fewer
  * splits than gemma4_qlinear_forward may choose, so the fp32 summation order, and with
  * it the last bits of some outputs, can differ from that call's; unsplit bf16-form
- * plans on the 64- and 128-row tiles need none), so no call is refused for want of
+ * plans on tiles of 32 to 128 rows need none), so no call is refused for want of
  * scratch.  Every call
  * on a GPU shares that GPU's array: calls that overlap in time on one GPU (other
  * streams, other threads) race and must be serialized by the caller. */

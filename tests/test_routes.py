@@ -48,3 +48,12 @@ def test_pinned_path_plans_freely():
     r = route(8192, 3840, 17, min_rows=1)
     assert not r["decode"] and r["splits"] > 1 and r["scratch"] > 0
     assert route(15360, 3840, 700, min_rows=1 << 20)["decode"]
+
+
+def test_tiles_of_shapes_the_kpair_tiles_cannot_address():
+    """Outputs of millions of columns run on the 128-row tile at any row count (the offsets
+    of the kpair tiles are 32 bits)."""
+    for m in (1, 40, 64, 200):
+        r = route(5_000_000, 64, m, min_rows=1)
+        assert not r["decode"] and not r["kpair"] and r["bm"] in (128, 256), r
+    assert route(4_000_000, 64, 40, min_rows=1)["kpair"]
