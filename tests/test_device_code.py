@@ -1,6 +1,6 @@
 """Checks on the compiled gfx950 code (CPU only: hipcc cross-compiles).
 
-The GEMM issues its LDS DMAs (`buffer_load_dwordx4 ... lds`) from inline asm, which
+The GEMMs issue their LDS DMAs (`buffer_load_dwordx4 ... lds`) from inline asm, which
 the compiler's hazard recognizer cannot see into.  A VALU write of an SGPR (for
 example a `v_readlane` reloading a spilled resource or offset SGPR) needs 5 wait
 states before a vector memory instruction reads that SGPR; the asm supplies them
@@ -18,8 +18,8 @@ from helios_amd import build as hbuild
 WAIT_STATES = 5
 
 
-def _kernels(asm: str):
-    for m in re.finditer(r"\n(_ZN\S*gemm_kernel\S*):[^\n]*\n", asm):
+def _kernels(asm: str, kernel: str = "gemm_kernel"):
+    for m in re.finditer(rf"\n(_ZN\S*{kernel}\S*):[^\n]*\n", asm):
         body = asm[m.end():asm.index("s_endpgm", m.end())]
         lines = [l.strip() for l in body.splitlines()
                  if l.strip() and not l.strip().startswith((";", "."))]
@@ -46,6 +46,12 @@ def kpair_asm():
     return hbuild.device_asm("q4_gemm_kpair.hip")
 
 
+def test_kpair_dma_sgpr_hazards_covered(kpair_asm):
+    kernels = list(_kernels(kpair_asm, "kpair_kernel"))
+    assert len(kernels) == 6  # tiles of 32, 48, .. 112 rows
+    _check_dma_hazards(kernels)
+
+
 def test_lds_dma_sgpr_hazards_covered(gemm_asm):
     kernels = list(_kernels(gemm_asm))
     # bf16 / fp32 outputs, bf16 / fp32 GeGLU pairs, bf16 / fp32 outputs with a LoRA
@@ -54,6 +60,10 @@ def test_lds_dma_sgpr_hazards_covered(gemm_asm):
     assert len(kernels) == 30
     assert sum("ELi256ELi256ELi1E" in name for name, _ in kernels) == 6
     assert sum("ELi256ELi2E" in name for name, _ in kernels) == 12
+    _check_dma_hazards(kernels)
+
+
+def _check_dma_hazards(kernels):
     for name, lines in kernels:
         dmas = 0
         for i, line in enumerate(lines):
@@ -75,13 +85,24 @@ def test_lds_dma_sgpr_hazards_covered(gemm_asm):
         assert dmas > 0, name
 
 
-def test_no_spills_and_lds_budget(gemm_asm):
+@pytest.mark.parametrize("asm", ["gemm_asm", "kpair_asm"])
+def test_no_spills_and_lds_budget(asm, request):
     # scratch spills would be VMEM loads counted by the kernel's manual vmcnt waits
+    asm = request.getfixturevalue(asm)
     for field in ("vgpr_spill_count", "private_segment_fixed_size"):
-        vals = [int(v) for v in re.findall(rf"\.{field}:\s+(\d+)", gemm_asm)]
-        assert vals and max(vals) == 0, (field, vals)
-    lds = [int(v) for v in re.findall(r"\.group_segment_fixed_size:\s+(\d+)", gemm_asm)]
+        vals = [int(v) for v in re.findall(rf"\.{field}:\s+(\d+)", asm)]
+        assert len(vals) >= 6 and max(vals) == 0, (field, vals)
+    lds = [int(v) for v in re.findall(r"\.group_segment_fixed_size:\s+(\d+)", asm)]
     assert max(lds) <= 160 * 1024
+
+
+def test_kpair_register_budget(kpair_asm):
+    """Two waves per SIMD (one 512-thread workgroup per CU): at most 256 VGPRs, and all of
+    a step's words and accumulators in registers."""
+    meta = [(n, v, p) for n, v, p in _kernel_meta(kpair_asm) if "kpair_kernel" in n]
+    assert len(meta) == 6
+    for name, vgprs, private in meta:
+        assert private == 0 and vgprs <= 256, f"{name}: {vgprs} VGPRs"
 
 
 # --------------------------------------------------------------- LDS DMAs and barriers
