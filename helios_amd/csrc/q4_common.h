@@ -214,17 +214,6 @@ enum OutMode : int {
     kOutLoraF32 = 7,     // the same in fp32
 };
 
-// The LoRA delta a GEMM epilogue adds to its outputs (kOutLora*): t = x . A^T as
-// `slices` fp32 partial planes [slices][M][rank] (summed in slice order), B [N][rank]
-// fp32, the adapter's scale; rank a multiple of 4, at most 32.
-struct LoraEpilogue {
-    const float* part;
-    const float* b;
-    int rank;
-    int slices;
-    float scale;
-};
-
 // Where and how a decode kernel writes its outputs.
 struct OutParams {
     void* y;                   // y [M, N], h [M, F], or the greedy modes' logits [M, N] (may be null)

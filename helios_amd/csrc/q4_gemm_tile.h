@@ -1,8 +1,9 @@
-// Device pieces shared by the prefill GEMM kernels (q4_gemm.hip, q4_gemm_slab.hip): the
+// Device pieces shared by the prefill GEMM kernels (q4_gemm.hip, q4_gemm_kpair.hip): the
 // bias term's MFMA operands, the tile order and the LoRA epilogue.
 #pragma once
 
 #include "q4_common.h"
+#include "q4_kernels.h"
 
 namespace q4 {
 namespace {

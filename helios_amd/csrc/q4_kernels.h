@@ -7,7 +7,16 @@
 
 namespace q4 {
 
-struct LoraEpilogue;
+// The LoRA delta a GEMM epilogue adds to its outputs (kOutLora*): t = x . A^T as
+// `slices` fp32 partial planes [slices][M][rank] (summed in slice order), B [N][rank]
+// fp32, the adapter's scale; rank a multiple of 4, at most 32.
+struct LoraEpilogue {
+    const float* part;
+    const float* b;
+    int rank;
+    int slices;
+    float scale;
+};
 
 // Weight records: one per (16-row block, group pair), [row block][pair], 1152 bytes
 // each: the 1 KiB tile of tiled words (uint4 per lane) and then the block's 16 scale/

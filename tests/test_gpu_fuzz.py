@@ -4,7 +4,7 @@ Each projection case draws N (or F for a gate|up pair), K (a multiple of 64), M 
 row ranges (0, 1, 2, 3-4, 5-16, 17-31, 32-64, 65-300; GEMM cases also 300-2100), 4 or 8 bits, a bf16 or fp32
 output, and the automatic path choice or the GEMM pinned from 32 rows.  Between them
 the cases reach every decode variant (row, per-row-block, streaming, global-x; 16-row
-slabs), the GEMM's 256-, 128- and 64-row tiles with and without a K split, and the
+slabs), the GEMM's 256- and 128-row and kpair tiles with and without a K split, and the
 ragged edges (N not a multiple of 16, K not a multiple of 128, a last row block or
 group pair partly empty).  Sampled rows are checked with the bars of
 test_gpu_parity.py (bf16 max |err| <= 1e-2 RMS + ulp/2, fp32 <= 2e-3 RMS) and, for
@@ -48,7 +48,7 @@ def _cases(count=40, seed=20261202):
 
 
 def _gemm_cases(count=16, seed=20261203):
-    """Cases on the GEMM: M of 32-300 rows (half of them <= 64: the 64-row tile), the
+    """Cases on the GEMM: M of 32-300 rows (half of them <= 64), the
     GEMM pinned, pairs more often."""
     rng = np.random.default_rng(seed)
     cases = []
@@ -66,7 +66,7 @@ def _gemm_cases(count=16, seed=20261203):
 
 
 def _gemm_cases_tall(count=8, seed=20261209):
-    """The GEMM at 300-2100 rows (the 64-row tile unsplit or split, the 128- and
+    """The GEMM at 300-2100 rows (kpair tiles unsplit or split, the 128- and
     256-row tiles; N up to 3000 keeps the oracle rows cheap)."""
     rng = np.random.default_rng(seed)
     cases = []

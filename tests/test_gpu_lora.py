@@ -99,9 +99,9 @@ def test_lora_adapter_directory(gpu_lib, tmp_path):
 
 
 # Prefill shapes whose GEMM plan is unsplit (gate at 2048 rows on 256-row tiles, k at
-# 2048 and the full-attention q at 512 on 64-row tiles): the GEMM's epilogue adds the
-# delta (t staged in LDS, fp32 matrix cores for t . B^T, then lora_up's rounding
-# steps).  Ranks that are multiples of 4 up to 32 take it; 48 and 64 (past 32) and 6
+# 2048 and the full-attention q at 512 on kpair tiles of 64 rows; not the 8-bit k): the
+# GEMM's epilogue adds the delta (t staged in LDS, fp32 matrix cores for t . B^T, then
+# lora_up's rounding steps).  Ranks that are multiples of 4 up to 32 take it; 48 and 64 (past 32) and 6
 # (not a multiple of 4) the LoRA kernels after the forward.  Sampled rows against the
 # oracle, same bars.
 @pytest.mark.parametrize("n,k,m,r,bits", [(15360, 3840, 2048, 16, 4), (2048, 3840, 2048, 4, 4),

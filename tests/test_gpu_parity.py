@@ -453,7 +453,7 @@ def test_forward_decode_slabs_past_32_rows(gpu_lib, proj, m):
 
 @pytest.mark.parametrize("m", [33, 64])
 def test_gemm_short_prompt_mlp(gpu_lib, gemm_from_32, m):
-    """Short prompts and prefill tails on the MLP shapes (the 64-row tile): gate and
+    """Short prompts and prefill tails on the MLP shapes (kpair tiles of 32 to 64 rows, K split): gate and
     down on sampled rows against the oracle (the gate|up pair: test_gpu_geglu.py)."""
     import torch
 
@@ -475,10 +475,9 @@ def test_gemm_short_prompt_mlp(gpu_lib, gemm_from_32, m):
 
 @pytest.mark.parametrize("proj,m", [("q_proj", 80), ("o_proj", 113), ("q_proj", 128), ("full_q_proj", 128),
                                     ("full_o_proj", 128)])
-def test_gemm_64_row_tile_two_row_tiles(gpu_lib, gemm_from_32, proj, m):
-    """The 64-row tile past 64 rows (two row tiles, the second ragged at 80 and 113):
-    the attention projections at 65-128 rows; sampled rows of both tiles against the
-    oracle."""
+def test_gemm_several_row_tiles(gpu_lib, gemm_from_32, proj, m):
+    """Two to four row tiles (kpair, 32 or 64 rows, the last one ragged at 80 and 113),
+    K split: the attention projections at 65-128 rows; sampled rows against the oracle."""
     import torch
 
     shapes = {**PROJ, **FULL_ATTENTION}
@@ -499,16 +498,13 @@ def test_gemm_64_row_tile_two_row_tiles(gpu_lib, gemm_from_32, proj, m):
     assert assert_close(yf[rt], want, f"{proj} m={m} f32") < 5e-4
 
 
-# (N, M) whose plans (64-row tile, 8 splits; 64-row, 4 splits; 128-row, 4 splits;
-# 256-row, 3 splits) end a K split of two or more octets on the last octet
+# kpair tiles of 32, 48, 32 and 80 rows in 8, 4, 1 and 1 splits (every tile with such a
+# last octet: test_gpu_forced_plans.py)
 @pytest.mark.parametrize("n,m", [(1000, 40), (1000, 700), (1000, 1500), (3000, 1500)])
 def test_gemm_last_octet_of_one_group(gpu_lib, gemm_from_32, n, m):
-    """K of 57 groups: seven whole octets and a last octet of one group.  Where a K
-    split ends on it with two or more octets, that octet's one step also applies the
-    previous octet's bias term, so the 64- and 128-row tiles write its group sums of x
-    after the loop and the 256-row tile loads them there from the pre-pass; with eight
-    splits the octet is a split of its own.  Sampled rows against the oracle, bf16 and
-    fp32."""
+    """K of 57 groups: seven whole octets and a last octet of one group (a last step of one
+    group of four); with eight splits the octet is a split of its own.  Sampled rows against
+    the oracle, bf16 and fp32."""
     import torch
 
     k = 57 * 64
