@@ -906,14 +906,16 @@ __global__ void split_geglu_kernel(const float* __restrict__ part, void* __restr
 //   + for a split: kSplitUs + kPerSplitUs per split + the partial sums' bytes
 //   + for a pre-pass (the 256-row tile's X_g; x16 in its forms): kPrePassUs and x16's bytes,
 // and the cheapest wins.  The fill term is the clock and the memory shared by more
-// workgroups.  The constants are fitted (least squares of the logarithm) to every plan
-// within 1.5x of the best of its case, measured as forwards in a graph over rotated
-// weight copies on five shapes (qkv 8192x3840, o 3840x4096, down 3840x15360, k 2048x3840,
-// the gate|up pair 30720x3840) at fourteen row counts from 20 to 1600, every tile with 1,
-// 2, 3, 4, 5 and 8 splits: the picks average 0.2% and at worst 4.7% over the fastest of
-// those plans.  (The constants before, without the kpair tiles, chose up to 46% slower
-// than the best tile of their own at those sizes: the pair at 1100 rows 413 us against
-// 330 on the 64-row tile, and 282 on a kpair tile of 112 rows.)
+// workgroups.  The constants are fitted to plans measured as forwards in a graph over
+// rotated weight copies, bf16 outputs: thirteen 4-bit shapes (N 1024 to 30720, K 1024 to
+// 15360) at 33 row counts from 32 to 2500, every tile and form with 1 to 15 splits that is
+// within reach of the best (429 cases).  The picks average 0.3% over the fastest plan of
+// their case and at worst 10.6% (8280x6720 at 1700 rows, where the fp16 form would win: the
+// fit holds that form back outside the widest outputs); none is more than 3% behind what the
+// plan took before the kpair tiles.  (Fitted to five shapes
+// of K = 3840 to 15360 up to 1600 rows the constants gave 0.8% and 15.8% here, and up to 6%
+// behind the plans before: 8280x6720 at 1432 rows 187 us on 96-row tiles against 177 on
+// 256, 11000x1024 at 1200 43.4 us in the fp16 form against 41.4.)
 namespace {
 struct TileShape {
     int bm, bn;
@@ -926,31 +928,35 @@ struct TileShape {
 // 107 against 85 and 331 against 282) and is gone.
 constexpr TileShape kTileShapes[] = {{256, 256, false}, {128, 256, false}, {32, 256, true}, {48, 256, true},
                                      {64, 256, true},   {80, 256, true},   {96, 256, true}, {112, 256, true}};
-constexpr double kFill = 0.426;
-constexpr double kSplitUs = 3.8, kPerSplitUs = 0.38;  // a split's reduction launch
-constexpr double kPartialBytesPerUs = 17.0e6;         // partial sums written and read back, mostly in the caches
+constexpr double kFill = 0.384;
+constexpr double kSplitUs = 3.61, kPerSplitUs = 0.36;  // a split's reduction launch
+constexpr double kPartialBytesPerUs = 9.56e6;         // partial sums written and read back, mostly in the caches
 // and past what those take (the 8-bit pair at 700 rows split in two, 172 MB: its reduction
 // 35 us, where the cached rate says 10)
 constexpr double kPartialCached = 64.0e6, kPartialFarBytesPerUs = 6.7e6;
-constexpr double kPrePassUs = 3.0;                    // a pre-pass launch
+constexpr double kPrePassUs = 4.71;                   // a pre-pass launch
 // a workgroup's time over `groups` groups, alone on its CU
 double body_us(const TileShape& ts, double step_scale, int groups) {
     if (ts.kpair) {
         const double mt = ts.bm / 16;
-        return groups / 4.0 * (0.693 + 0.261 * mt) + 0.737 * mt;
+        return groups / 4.0 * (0.914 + 0.2085 * mt) + 0.973 * mt;
     }
-    const double step = ts.bm == 256 ? 1.202 : 0.766;
-    return groups * step * step_scale + 1.464 * (1.0 + ts.bm / 64.0);
+    return ts.bm == 256 ? groups * 1.144 * step_scale + 8.13 : groups * 0.757 + 6.08;
 }
-// the fp16 form: its group step against the bf16 form's (gate 15360x3840 at 2048 rows,
-// the kernel alone, steady clock: 210-215 vs 218-223 us), and its pre-pass's extra
-// time per byte of x16 (12.3 us against the group-sum pre-pass's 5.0 for 15.7 MB)
-constexpr double kF16StepScale = 0.95;
-constexpr double kPrepBytesPerUs = 2.15e6;
-// one-pass 8-bit: its group step (over K, not 2K) against the 4-bit tile's of the
-// same height (8-bit gate 15360x3840 at 2048 rows with the pre-pass: 262 us on 256-row
-// tiles, 120 steps per CU: 1.16; 325 on 128-row tiles, 240 steps: 1.19)
-constexpr double kQ8StepScale = 1.2;
+// the fp16 form: its group step against the bf16 form's, and what its pre-pass takes over
+// the group-sum pre-pass, per launch and per byte of x16 (alone, gate 15360x3840 at 2048
+// rows: the kernel 210-215 us against 218-223, the pre-pass 12.3 against 5.0 for 15.7 MB)
+constexpr double kF16StepScale = 0.92;
+constexpr double kPrepUs = 1.4, kPrepBytesPerUs = 1.88e6;
+// One-pass 8-bit: constants of its own, fitted to its plans on seven 8-bit shapes at
+// seventeen row counts from 40 to 2048 beside the kpair plans there.  With the 4-bit
+// tiles' constants and a common factor on the step the plan took 256-row tiles in two
+// splits where 128 rows unsplit are 3-5% ahead (qkv at 700 rows 84.4 us against 81.7, the
+// pair at 200 92.1 against 87.6, k at 2048 67.6 against 64.8).
+constexpr double kQ8Step256 = 1.615, kQ8Step128 = 1.0;  // us a group step (over K, not 2K)
+constexpr double kQ8Fill = 0.15;
+constexpr double kQ8SplitUs = 7.1, kQ8PartialBytesPerUs = 4.3e6;
+constexpr double kQ8PrepUs = 1.0;
 size_t round256(size_t b) { return (b + 255) & ~(size_t)255; }
 }  // namespace
 
@@ -1013,14 +1019,19 @@ GemmPlan plan_gemm(int m, const Layout& l, size_t max_workspace) {
                 const size_t part = s > 1 ? (size_t)s * m * l.n * 4 : 0;
                 if (part > kMaxPartialBytes) break;
                 if (xa + x16 + rexp + part > max_workspace) break;  // (more splits need more)
+                const bool q8 = form == 2;
                 const double wgs = (double)(tiles * s);
                 const double rounds = (double)((tiles * s + cus - 1) / cus);
-                const double scale = form == 1 ? kF16StepScale : form == 2 ? kQ8StepScale : 1.0;
                 const int gs = per * 8 < groups ? per * 8 : groups;
-                const double t = rounds * body_us(ts, scale, gs) * (1.0 + kFill * wgs / (rounds * cus)) +
-                                 (s > 1 ? kSplitUs + kPerSplitUs * s + part / kPartialBytesPerUs : 0.0) +
+                const double body = q8 ? gs * (bm == 256 ? kQ8Step256 : kQ8Step128)
+                                       : body_us(ts, form == 1 ? kF16StepScale : 1.0, gs);
+                const double t = rounds * body * (1.0 + (q8 ? kQ8Fill : kFill) * wgs / (rounds * cus)) +
+                                 (s > 1 ? (q8 ? kQ8SplitUs : kSplitUs) + kPerSplitUs * s +
+                                              part / (q8 ? kQ8PartialBytesPerUs : kPartialBytesPerUs)
+                                        : 0.0) +
                                  (part > kPartialCached ? (part - kPartialCached) / kPartialFarBytesPerUs : 0.0) +
-                                 ((bm == 256 || pre) ? kPrePassUs + x16 / kPrepBytesPerUs : 0.0);
+                                 (bm == 256 || pre ? kPrePassUs : 0.0) +
+                                 (pre ? (q8 ? kQ8PrepUs : kPrepUs) + x16 / kPrepBytesPerUs : 0.0);
                 if (best < 0.0 || t < best) {
                     best = t;
                     p.bm = bm;

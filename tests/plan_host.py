@@ -24,7 +24,8 @@ def _load():
         if not os.path.exists(SO) or any(os.path.getmtime(d) > os.path.getmtime(SO) for d in deps):
             os.makedirs(os.path.dirname(SO), exist_ok=True)
             subprocess.run(["g++", "-std=c++17", "-O1", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
-                            "-I", hbuild.CSRC, deps[0], hbuild.LIB_PATH, "-o", SO], check=True, capture_output=True)
+                            "-I", hbuild.CSRC, deps[0], "-L", hbuild.LIB_DIR, "-l:" + hbuild.LIB_NAME,
+                            "-Wl,-rpath,$ORIGIN/../../helios_amd/lib", "-o", SO], check=True, capture_output=True)
         _fn = ctypes.CDLL(SO)
         i, p, ul = ctypes.c_int, ctypes.c_void_p, ctypes.c_ulong
         _fn.q4_route.argtypes = [i] * 7 + [ul, ctypes.POINTER(ctypes.c_long)]

@@ -498,7 +498,7 @@ def test_gemm_several_row_tiles(gpu_lib, gemm_from_32, proj, m):
     assert assert_close(yf[rt], want, f"{proj} m={m} f32") < 5e-4
 
 
-# kpair tiles of 32, 48, 32 and 80 rows in 8, 4, 1 and 1 splits (every tile with such a
+# kpair tiles of 32, 48, 48 and 80 rows in 8, 4, 2 and 1 splits (every tile with such a
 # last octet: test_gpu_forced_plans.py)
 @pytest.mark.parametrize("n,m", [(1000, 40), (1000, 700), (1000, 1500), (3000, 1500)])
 def test_gemm_last_octet_of_one_group(gpu_lib, gemm_from_32, n, m):
